@@ -541,3 +541,20 @@ def test_c5_conv_backward_properties(ctx):
         ref = oracle.col2im(gcol.astype(np.float32), 1, C, H, W, 3, 3, stride=1, pad=1)[0]
         den = oracle.col2im(gcol_abs.astype(np.float32), 1, C, H, W, 3, 3, stride=1, pad=1)[0]
         assert np.all(np.abs(gi[b] - ref) <= tol(9 * OC) * den * 1.01 + 1e-6), f"image {b}"
+
+
+@pytest.mark.parametrize("channels", [47, 48, 49])
+def test_col2im_both_kernels(ctx, channels):
+    """Around the channel count where zn_col2im (lanes along channels) takes over from zn_col2im_px (lanes along
+    pixels): both bit-identical to the reference's order."""
+    B, H, W, KH, KW, st, pd = 2, 9, 67, 3, 3, (2, 1), (1, 1)
+    OH, OW = (H + 2 - KH) // 2 + 1, (W + 2 - KW) // 1 + 1
+    rng = np.random.default_rng(channels)
+    col = uniform(rng, (B * OH * OW, KH * KW * channels))
+    dcol, dout = ctx.to_device(col), ctx.alloc(B * channels * H * W).fill(np.nan)
+    announce(f"col2im {channels} channels")
+    ctx.col2im(dcol, dout, B, channels, H, W, KH, KW, OH, OW, *st, *pd)
+    np.testing.assert_array_equal(dout.download().reshape(B, channels, H, W),
+                                  oracle.col2im(col, B, channels, H, W, KH, KW, stride=st, pad=pd))
+    for b in (dcol, dout):
+        b.close()

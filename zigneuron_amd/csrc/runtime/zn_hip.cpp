@@ -62,16 +62,20 @@ constexpr TileShape kTiles[kNumTiles] = {{256, 128, 16, 512, "x", true, true, tr
                                          {32, 32, 32, 64, "s", true, false, true},
                                          {128, 128, 32, 512, "r", false, false, true},
                                          {64, 64, 16, 256, "h", false, false, true},
-                                         {256, 256, 16, 512, "w", false, false, false}};
+                                         {256, 256, 16, 512, "w", false, false, false},
+                                         {256, 256, 32, 512, "sw", false, false, true},
+                                         {256, 128, 32, 512, "sx", false, false, true},
+                                         {128, 128, 32, 512, "sr", false, false, true},
+                                         {128, 64, 32, 256, "sn", false, false, true}};
 constexpr const char *kLayoutName[3] = {"nn", "nt", "tn"};
 
-enum EltKernel { kFill, kCopy, kAddBias, kActFwd, kActBwd, kAccBias, kIm2col, kSoftmax, kCol2im, kRowSum, kDenseGrad, kRegroup, kPack, kToNhwc, kHold, kNumElt };
+enum EltKernel { kFill, kCopy, kAddBias, kActFwd, kActBwd, kAccBias, kIm2col, kSoftmax, kCol2im, kRowSum, kDenseGrad, kRegroup, kPack, kToNhwc, kHold, kCol2imPx, kNumElt };
 constexpr const char *kEltName[kNumElt] = {"zn_fill_f32",        "zn_copy_f32", "zn_add_bias",
                                            "zn_activation_forward", "zn_activation_backward",
                                            "zn_accumulate_bias", "zn_im2col",   "zn_softmax_rows",
                                            "zn_col2im",          "zn_row_sum",  "zn_dense_grad_prologue",
                                            "zn_weight_regroup", "zn_pack_rows", "zn_nchw_to_nhwc",
-                                           "zn_hold_stream"};
+                                           "zn_hold_stream",     "zn_col2im_px"};
 
 constexpr const char *kGemmObject = "zn_gemm_gfx950.hsaco";
 constexpr const char *kConvObject = "zn_conv_gfx950.hsaco";
@@ -2185,7 +2189,9 @@ static ZnIm2colArgs col_args(float *image, float *col, int64_t batch, int64_t c,
 }
 
 // zn_im2col: one workgroup per tile of 64 col rows x 64 taps; zn_col2im: one
-// per 64 pixels of an input row (grid-stride loops cover the rest).
+// per 64 pixels of an input row (grid-stride loops cover the rest), or below
+// kCol2imChannels channels one thread per input element (zn_col2im_px).
+constexpr int kCol2imChannels = 48;
 static int im2col_launch(zn_ctx *ctx, const ZnIm2colArgs &a) {
     const int rc = select_device(ctx);
     if (rc) return rc;
@@ -2199,9 +2205,13 @@ static int col2im_launch(zn_ctx *ctx, const ZnIm2colArgs &a) {
     const int rc = select_device(ctx);
     if (rc) return rc;
     const int64_t cap = cus_now(ctx) * 32;
+    ZnIm2colArgs c = a;
+    if (a.channels < kCol2imChannels) {
+        const int64_t blocks = std::min<int64_t>(cdiv((int64_t)a.batch * a.channels * a.in_h * a.in_w, 256), cap);
+        return launch(ctx, ctx->elt[kCol2imPx], (unsigned)blocks, 1, 256, &c);
+    }
     const int64_t units = (int64_t)a.batch * a.in_h * cdiv(a.in_w, 64);
     const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>(units, cap));
-    ZnIm2colArgs c = a;
     return launch(ctx, ctx->elt[kCol2im], (unsigned)blocks, 1, 256, &c);
 }
 
