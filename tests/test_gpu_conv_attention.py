@@ -558,3 +558,52 @@ def test_col2im_both_kernels(ctx, channels):
                                   oracle.col2im(col, B, channels, H, W, KH, KW, stride=st, pad=pd))
     for b in (dcol, dout):
         b.close()
+
+
+@pytest.mark.parametrize("batch,seq,d", [(1, 1000, 80), (1, 2048, 64), (2, 321, 128), (1, 63, 33), (3, 257, 96),
+                                         (1, 255, 1), (70, 130, 64), (1, 4097, 32)])
+def test_attention_key_ranges(ctx, batch, seq, d):
+    """Few problems: the keys go to ranges of their own and zn_attention_combine merges them (and the shapes on either
+    side of that rule); within the bound of the fused walk."""
+    rng = np.random.default_rng(seq + d)
+    q, k, v = (uniform(rng, (batch, seq, d)) for _ in range(3))
+    scale = 1.0 / np.sqrt(d)
+    dq, dk, dv, do = ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), ctx.alloc(q.size).fill(np.nan)
+    announce(f"attention ranges {batch}x{seq}x{d}")
+    ctx.attention_forward(dq, dk, dv, do, batch, seq, d, scale)
+    out = do.download().reshape(q.shape)
+    for i in {0, batch - 1}:
+        exact, bound = attention_bound(q[i], k[i], v[i], scale)
+        assert np.all(np.abs(out[i] - exact) <= bound)
+    for b in (dq, dk, dv, do):
+        b.close()
+
+
+@pytest.mark.parametrize("batch,seq,d", [(1, 700, 64), (40, 200, 64), (1, 300, 100)])
+def test_attention_non_finite_and_huge(ctx, batch, seq, d):
+    """Scores of -inf (a key whose product with every query is -inf gets weight 0), a NaN key, and values of 1e30 (whose
+    scaled parts overflow): what fp32 arithmetic gives, on the queries they reach and on the others."""
+    rng = np.random.default_rng(seq)
+    q, k, v = (np.abs(uniform(rng, (batch, seq, d))) + np.float32(0.1) for _ in range(3))
+    k[0, 5] = -np.inf            # weight 0 for every query
+    v[0] *= np.float32(1e30)
+    if batch > 1:
+        k[1, seq - 1, 3] = np.nan  # every query of problem 1 is NaN
+        q[2, 17, 0] = np.nan       # one query of problem 2
+        v[3, 9, 2] = np.inf        # one head dim of problem 3
+    scale = 1.0 / np.sqrt(d)
+    dq, dk, dv, do = ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), ctx.alloc(q.size).fill(0.0)
+    announce(f"attention non-finite {batch}x{seq}x{d}")
+    ctx.attention_forward(dq, dk, dv, do, batch, seq, d, scale)
+    out = do.download().reshape(q.shape)
+    with np.errstate(all="ignore"):
+        for i in range(min(batch, 5)):
+            s = (q[i].astype(np.float64) @ k[i].astype(np.float64).T) * scale
+            e = np.exp(s - s.max(1, keepdims=True))
+            ref = (e @ v[i].astype(np.float64)) / e.sum(1, keepdims=True)
+            np.testing.assert_array_equal(np.isnan(out[i]), np.isnan(ref), err_msg=str(i))
+            np.testing.assert_array_equal(np.isinf(out[i]), np.isinf(ref), err_msg=str(i))
+            fin = np.isfinite(ref)
+            assert np.all(np.abs(out[i][fin] - ref[fin]) <= 1e-4 * np.abs(ref[fin])), i
+    for b in (dq, dk, dv, do):
+        b.close()

@@ -29,6 +29,9 @@
 #include "../zn_kernel_args.h"
 
 #include "zn_mfma_stage.h"
+#include "zn_split.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -199,6 +202,334 @@ __device__ __forceinline__ void attention_tile(const ZnAttnArgs &p) {
     }
 }
 
+// ---------------------------------------------------------------- split form
+// The same walk on the bf16 matrix cores, every operand value split into
+// three bf16 parts (zn_split.h): S^T = K . (cQ)^T and O^T += V^T . P^T on
+// v_mfma_f32_16x16x32_bf16.  Q is split once per workgroup into registers; K
+// and V blocks of 32 keys are loaded through registers, split and written to
+// LDS (two stages), V transposed on the way.  In the order of a slice used
+// here (chunk c: k = 4c .. 4c + 3 and 16 + 4c .. 16 + 4c + 3) the two 16-key
+// S^T accumulators of a lane are its chunk of the P^T operand, so P stays in
+// registers as before.
+//
+// A walk whose scores or sums are not finite (an Inf or NaN input, or
+// magnitudes whose scaled products overflow) is done again by its wave alone
+// on the fp32 matrix cores, straight from memory (attention_plain).
+//
+// Few problems leave most of the chip idle: then blockIdx.z takes a range of
+// the keys, and zn_attention_combine merges the ranges' (O, m, l).
+template <int DP, int NW, int FQ, int BKV>
+struct AttnSplit {
+    static constexpr int NT = NW * kWave;
+    static constexpr int SL = DP / 32, DB = DP / 16;  // 32-deep slices and 16-row blocks of the head dim
+    static constexpr int KB = BKV / 32;               // 32-key slices of a block
+    static constexpr int kPart = DP * 2 * BKV;        // bytes of one bf16 part of a K (or V) block
+    static constexpr int kStage = 6 * kPart;
+    static constexpr int kUnits = DP * BKV / 4;       // staging units of 8 values: K, then V
+    static constexpr int UPT = (kUnits + NT - 1) / NT;
+    static_assert(kUnits / 2 % kWave == 0, "a wave's units are all of K or all of V");
+
+    __device__ static __forceinline__ int slot(int r, int c) { return r * 64 + ((c ^ (-(r >> 2) & 3)) << 4); }
+    __device__ static __forceinline__ float max_over_quads(float x) {
+        // the 4 lanes of a query: li, li + 16, li + 32, li + 48
+        const auto a = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+        x = fmaxf(__builtin_bit_cast(float, a[0]), __builtin_bit_cast(float, a[1]));
+        const auto b = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+        return fmaxf(__builtin_bit_cast(float, b[0]), __builtin_bit_cast(float, b[1]));
+    }
+
+    __device__ static __forceinline__ void run(const ZnAttnArgs &p, char *lds) {
+        const int tid = threadIdx.x, lane = tid & (kWave - 1);
+        const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+        const int li = lane & 15, lh = lane >> 4;
+        const int S = p.seq_len, D = p.d_k;
+        const int64_t base = (int64_t)blockIdx.x * p.stride;
+        const int q0 = (int)blockIdx.y * (NW * FQ * 16) + wave * FQ * 16;
+        const int kbeg = (int)blockIdx.z * p.keys_per_split;
+        const int kend = min(S, kbeg + p.keys_per_split);
+        const uint32_t bytes = (uint32_t)((int64_t)S * D * 4);
+        const __amdgpu_buffer_rsrc_t rq = make_rsrc(p.q + base, bytes);
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(p.k + base, bytes);
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc(p.v + base, bytes);
+
+        // staging units of this thread: byte offset of the first load at key kbeg, LDS position
+        uint32_t off0[UPT];
+        int lpos[UPT];
+        bool is_v[UPT];
+#pragma unroll
+        for (int j = 0; j < UPT; ++j) {
+            const int u = j * NT + tid;
+            is_v[j] = __builtin_amdgcn_readfirstlane(u) >= kUnits / 2;
+            if (!is_v[j]) {
+                const int key = u / (DP / 8), dc = u % (DP / 8);  // chunk dc % 4 of slice dc / 4
+                const int d = 32 * (dc / 4) + 4 * (dc % 4);
+                off0[j] = (uint32_t)((kbeg + key) * D + d) * 4u;
+                lpos[j] = (dc / 4) * (BKV * 64) + slot(key, dc % 4);
+            } else {
+                const int v = u - kUnits / 2, d = v % DP, ks = v / DP / 4, c = v / DP % 4;  // key slice and chunk
+                off0[j] = d < D ? (uint32_t)((kbeg + 32 * ks + 4 * c) * D + d) * 4u : kOutOfRange;
+                lpos[j] = 3 * kPart + ks * (DP * 64) + slot(d, c);
+            }
+        }
+        const uint32_t row = (uint32_t)D * 4u;
+        float g[UPT][8];
+        auto load = [&](int b, int j) {
+            if (j * NT + tid >= kUnits) return;  // whole waves
+            const uint32_t off = off0[j] == kOutOfRange ? kOutOfRange : off0[j] + (uint32_t)b * (BKV * row);
+            if (!is_v[j]) {
+                const zn_f32x4 v0 = __builtin_bit_cast(zn_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 0));
+                const zn_f32x4 v1 = __builtin_bit_cast(zn_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 64, 0, 0));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    g[j][e] = v0[e];
+                    g[j][4 + e] = v1[e];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t o = off == kOutOfRange ? off : off + (e < 4 ? e : 12 + e) * row;
+                    g[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, o, 0, 0));
+                }
+            }
+        };
+        auto stage = [&](int st, int j) {
+            if (j * NT + tid >= kUnits) return;
+            zn_u32x4 w[3];
+            split8(g[j], w);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *reinterpret_cast<zn_u32x4 *>(lds + st * kStage + lpos[j] + q * kPart) = w[q];
+        };
+        const int fr = slot(li, lh);
+        auto read_k = [&](int st, int sl, int kb, int q) {
+            return __builtin_bit_cast(zn_bf16x8, *reinterpret_cast<const zn_u32x4 *>(lds + st * kStage + q * kPart + sl * (BKV * 64) + kb * (16 * 64) + fr));
+        };
+        auto read_v = [&](int st, int ks, int db, int q) {
+            return __builtin_bit_cast(zn_bf16x8, *reinterpret_cast<const zn_u32x4 *>(lds + st * kStage + (3 + q) * kPart + ks * (DP * 64) + db * (16 * 64) + fr));
+        };
+
+#pragma unroll
+        for (int j = 0; j < UPT; ++j) load(0, j);
+        // Q^T fragments: query 16f + li, chunk lh of slice sl, times scale * log2(e)
+        zn_bf16x8 qf[FQ][SL][3];
+#pragma unroll
+        for (int f = 0; f < FQ; ++f)
+#pragma unroll
+            for (int sl = 0; sl < SL; ++sl) {
+                const int q = q0 + 16 * f + li, d = 32 * sl + 4 * lh;
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int de = d + (e < 4 ? e : 12 + e);
+                    const uint32_t off = q < S && de < D ? (uint32_t)(q * D + de) * 4u : kOutOfRange;
+                    x[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rq, off, 0, 0)) * p.scale_log2;
+                }
+                zn_u32x4 w[3];
+                split8(x, w);
+#pragma unroll
+                for (int r = 0; r < 3; ++r) qf[f][sl][r] = __builtin_bit_cast(zn_bf16x8, w[r]);
+            }
+
+        zn_f32x4 o[FQ][DB];
+        float m[FQ], l[FQ];  // running maximum (log2 domain), this lane's share of the running sum
+#pragma unroll
+        for (int f = 0; f < FQ; ++f) {
+#pragma unroll
+            for (int d = 0; d < DB; ++d) o[f][d] = zn_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            m[f] = -INFINITY;
+            l[f] = 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < UPT; ++j) stage(0, j);
+        constexpr int kPA[6] = {2, 1, 0, 1, 0, 0}, kPB[6] = {0, 1, 2, 0, 1, 0};
+        const int nblk = (kend - kbeg + BKV - 1) / BKV;
+        // MASK: the range's last block, its missing keys get score -inf
+        auto block = [&](int b, auto mc) {
+            constexpr bool MASK = decltype(mc)::value;
+            const int st = b & 1;
+            __syncthreads();  // block b is in LDS; every wave is done with block b - 1
+#pragma unroll
+            for (int j = 0; j < UPT; ++j) load(b + 1, j);
+            zn_f32x4 s[FQ][2 * KB];
+#pragma unroll
+            for (int f = 0; f < FQ; ++f)
+#pragma unroll
+                for (int kb = 0; kb < 2 * KB; ++kb) s[f][kb] = zn_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int kp = 0; kp < KB; ++kp)
+#pragma unroll
+                for (int sl = 0; sl < SL; ++sl) {
+                    zn_bf16x8 kf[2][3];
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) kf[kb][q] = read_k(st, sl, 2 * kp + kb, q);
+#pragma unroll
+                    for (int pr = 0; pr < 6; ++pr)
+#pragma unroll
+                        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                            for (int f = 0; f < FQ; ++f)
+                                s[f][2 * kp + kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kb][kPA[pr]], qf[f][sl][kPB[pr]],
+                                                                                            s[f][2 * kp + kb], 0, 0, 0);
+                }
+            zn_bf16x8 pf[FQ][KB][3];
+            const int left = kend - kbeg - b * BKV;  // keys of this range from this block on
+#pragma unroll
+            for (int f = 0; f < FQ; ++f) {
+                float mb = -INFINITY;
+#pragma unroll
+                for (int kb = 0; kb < 2 * KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if (MASK && 16 * kb + 4 * lh + r >= left) s[f][kb][r] = -INFINITY;
+                        mb = fmaxf(mb, s[f][kb][r]);
+                    }
+                const float mn = fmaxf(m[f], max_over_quads(mb) * kSplitUnscale);
+                const float alpha = exp2_fast(m[f] - mn);
+                float rs = 0.0f;
+#pragma unroll
+                for (int kb = 0; kb < 2 * KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        s[f][kb][r] = exp2_fast(__builtin_fmaf(s[f][kb][r], kSplitUnscale, -mn));
+                        rs += s[f][kb][r];
+                    }
+                l[f] = l[f] * alpha + rs;
+                m[f] = mn;
+                if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+                    for (int d = 0; d < DB; ++d) o[f][d] *= alpha;
+                }
+#pragma unroll
+                for (int ks = 0; ks < KB; ++ks) {
+                    float e8[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) e8[e] = s[f][2 * ks + e / 4][e % 4];
+                    zn_u32x4 w[3];
+                    split8(e8, w);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) pf[f][ks][q] = __builtin_bit_cast(zn_bf16x8, w[q]);
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < DB; ++d) {
+#pragma unroll
+                for (int ks = 0; ks < KB; ++ks) {
+                    zn_bf16x8 vf[3];
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) vf[q] = read_v(st, ks, d, q);
+#pragma unroll
+                    for (int pr = 0; pr < 6; ++pr)
+#pragma unroll
+                        for (int f = 0; f < FQ; ++f)
+                            o[f][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[kPA[pr]], pf[f][ks][kPB[pr]], o[f][d], 0, 0, 0);
+                }
+                // the next block's staging, spread over the products
+#pragma unroll
+                for (int j = 0; j < UPT; ++j)
+                    if (j * DB / UPT == d) stage(st ^ 1, j);
+            }
+        };
+        const int nfull = (kend - kbeg) / BKV;
+        for (int b = 0; b < nfull; ++b) block(b, std::false_type());
+        if (nfull < nblk) block(nfull, std::true_type());
+        bool bad = false;
+#pragma unroll
+        for (int f = 0; f < FQ; ++f) {
+            bad |= !(l[f] < INFINITY);
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    bad |= !(__builtin_fabsf(o[f][d][r]) < INFINITY);
+                    o[f][d][r] *= kSplitUnscale;
+                }
+        }
+        if (__builtin_amdgcn_ballot_w64(bad)) plain(p, rq, rk, rv, q0, kbeg, kend, lane, o, m, l);
+#pragma unroll
+        for (int f = 0; f < FQ; ++f) {
+            float sum = l[f] + __shfl_xor(l[f], 16);
+            sum += __shfl_xor(sum, 32);
+            const int q = q0 + 16 * f + li;
+            if (q >= S) continue;
+            if (p.splits > 1) {
+                // [problem][query][range]: D rounded up to 4 of O, then m and l
+                const int ld = ((D + 3) & ~3) + 4;
+                float *dst = p.part + (((int64_t)blockIdx.x * S + q) * p.splits + blockIdx.z) * ld;
+#pragma unroll
+                for (int d = 0; d < DB; ++d)
+                    if (16 * d + 4 * lh < D) *reinterpret_cast<zn_f32x4 *>(dst + 16 * d + 4 * lh) = o[f][d];
+                if (lh == 0) {
+                    dst[ld - 4] = m[f];
+                    dst[ld - 3] = sum;
+                }
+                continue;
+            }
+            float *orow = p.out + base + (int64_t)q * D;
+#pragma unroll
+            for (int d = 0; d < DB; ++d) {
+                const int col = 16 * d + 4 * lh;
+                if (col + 4 <= D) {
+                    *reinterpret_cast<zn_f32x4u *>(orow + col) = o[f][d] / sum;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (col + r < D) orow[col + r] = o[f][d][r] / sum;
+                }
+            }
+        }
+    }
+
+    // The wave's queries on the fp32 matrix cores, 16 keys at a time, K and V read from memory.
+    __device__ static __forceinline__ void plain(const ZnAttnArgs &p, __amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rk,
+                                                 __amdgpu_buffer_rsrc_t rv, int q0, int kbeg, int kend, int lane,
+                                                 zn_f32x4 (&o)[FQ][DB], float (&m)[FQ], float (&l)[FQ]) {
+        const int li = lane & 15, lh = lane >> 4;
+        const int S = p.seq_len, D = p.d_k;
+        auto get = [&](__amdgpu_buffer_rsrc_t r, int x, int d, int lim) {
+            const uint32_t off = x < lim && d < D ? (uint32_t)(x * D + d) * 4u : kOutOfRange;
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+        };
+#pragma unroll
+        for (int f = 0; f < FQ; ++f) {
+            const int q = q0 + 16 * f + li;
+#pragma unroll
+            for (int d = 0; d < DB; ++d) o[f][d] = zn_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            m[f] = -INFINITY;
+            l[f] = 0.0f;
+            for (int k0 = kbeg; k0 < kend; k0 += 16) {
+                zn_f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+                for (int d = 0; d < D; d += 4)
+                    s = __builtin_amdgcn_mfma_f32_16x16x4f32(get(rk, k0 + li, d + lh, kend), get(rq, q, d + lh, S) * p.scale_log2, s, 0, 0, 0);
+                float mb = -INFINITY;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (k0 + 4 * lh + r >= kend) s[r] = -INFINITY;
+                    mb = fmaxf(mb, s[r]);
+                }
+                const float mn = fmaxf(m[f], max_over_quads(mb));
+                const float ref = mn == -INFINITY ? 0.0f : mn;  // nothing but -inf scores so far
+                const float alpha = exp2_fast(m[f] - ref);
+                float rs = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    s[r] = exp2_fast(s[r] - ref);
+                    rs += s[r];
+                }
+                l[f] = l[f] * alpha + rs;
+                m[f] = mn;
+#pragma unroll
+                for (int d = 0; d < DB; ++d) {
+                    o[f][d] *= alpha;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)  // k index lh of step r: key k0 + 4 lh + r
+                        o[f][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(get(rv, k0 + 4 * lh + r, 16 * d + li, kend), s[r], o[f][d], 0, 0, 0);
+                }
+            }
+        }
+    }
+};
+
 }  // namespace
 
 // zn_attention_d<DP>[_v]: head dims up to DP (zero-padded), 4 waves = 128
@@ -215,3 +546,59 @@ __device__ __forceinline__ void attention_tile(const ZnAttnArgs &p) {
 ZN_ATTN_DIM(32, 64)
 ZN_ATTN_DIM(64, 64)
 ZN_ATTN_DIM(128, 32)
+
+// zn_attention_s<DP>: the split form, head dims up to DP, any alignment;
+// NW waves of FQ x 16 queries.
+#define ZN_ATTN_SPLIT(DP, NW, FQ, BKV)                                                                         \
+    extern "C" __global__ __launch_bounds__(NW * 64, 2) void zn_attention_s##DP(ZnAttnArgs p) {           \
+        typedef AttnSplit<DP, NW, FQ, BKV> T;                                                                  \
+        __shared__ __attribute__((aligned(1024))) char lds[2 * T::kStage];                                \
+        T::run(p, lds);                                                                                   \
+    }
+ZN_ATTN_SPLIT(32, 4, 2, 64)
+ZN_ATTN_SPLIT(64, 8, 2, 64)
+ZN_ATTN_SPLIT(96, 8, 1, 32)
+ZN_ATTN_SPLIT(128, 8, 1, 32)
+
+// out[query] = sum over ranges z of 2^(m_z - M) O_z / sum of 2^(m_z - M) l_z,
+// M = max m_z, the ranges in ascending order.  One wave per query: lane z
+// takes range z's m and l, lane d the head dims d and d + 64, whose range
+// loads are all independent (splits <= 32; MI355X, 1000 queries of 80 dims in
+// 16 ranges: one thread per element walking m, l and O took 12 us).
+constexpr int kMaxAttnSplits = 32;
+extern "C" __global__ __launch_bounds__(256) void zn_attention_combine(ZnAttnArgs p) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t q = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
+    if (q >= (int64_t)p.batch * p.seq_len) return;
+    const int ld = ((p.d_k + 3) & ~3) + 4;
+    const float *src = p.part + q * p.splits * ld;
+    float ov[2][kMaxAttnSplits];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int z = 0; z < kMaxAttnSplits; ++z) {
+            ov[i][z] = 0.0f;
+            if (z < p.splits && lane + 64 * i < p.d_k) ov[i][z] = src[z * ld + lane + 64 * i];
+        }
+    const bool in = lane < p.splits;
+    const float m = in ? src[lane * ld + ld - 4] : -INFINITY;
+    const float l = in ? src[lane * ld + ld - 3] : 0.0f;
+    float mx = m;
+#pragma unroll
+    for (int s = 1; s < kMaxAttnSplits; s <<= 1) mx = fmaxf(mx, __shfl_xor(mx, s));
+    const float w = exp2_fast(m - (mx == -INFINITY ? 0.0f : mx));
+    const float wl = in ? w * l : 0.0f;
+    float sum = 0.0f, o[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int z = 0; z < kMaxAttnSplits; ++z)
+        if (z < p.splits) {
+            const float wz = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), z));
+            sum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wl), z));
+            o[0] += wz * ov[0][z];
+            o[1] += wz * ov[1][z];
+        }
+    float *row = p.out + q / p.seq_len * p.stride + q % p.seq_len * p.d_k;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (lane + 64 * i < p.d_k) row[lane + 64 * i] = o[i] / sum;
+}

@@ -85,6 +85,10 @@ constexpr const char *kAttnObject = "zn_attention_gfx950.hsaco";
 // Fused attention kernels by padded head dim (zn_attention_d<dim>[_v]).
 constexpr int kAttnDims[3] = {32, 64, 128};
 constexpr int kAttnQueries = 128;  // queries per workgroup (4 waves x 32)
+// The split form (zn_attention_s<dim>): padded head dims, threads and queries of a workgroup.
+constexpr int kAttnSplitDims[4] = {32, 64, 96, 128};
+constexpr unsigned kAttnSplitThreads[4] = {256, 512, 512, 512};
+constexpr int kAttnSplitQueries[4] = {128, 256, 128, 128};
 
 struct ScratchDevice;
 
@@ -165,6 +169,8 @@ struct zn_ctx {
     int pair_fwd_threads[2] = {};              // its workgroup size (the kernel's launch bounds)
     hipFunction_t pair_bwd[4][2][2] = {};      // fused two-layer Dense backward [lower act][non-linear head][16-byte]
     hipFunction_t attn[3][2] = {};             // fused attention [head dim 32/64/128][16-byte I/O]
+    hipFunction_t attn_split[4] = {};          // the split form [head dim 32/64/96/128]
+    hipFunction_t attn_combine = nullptr;      // merges its key ranges
     hipFunction_t gemm[3][kNumTiles][3] = {};  // [layout][tile][staging: 4-byte, 16-byte, 16-byte unaligned (r only)]
     int gemm_threads[3][kNumTiles][3] = {};    // their workgroup sizes (the kernels' launch bounds)
     hipFunction_t conv[kNumTiles][2][2] = {};  // implicit-GEMM convolution [tile][16-byte W rows][4-pixel gather]
@@ -1768,6 +1774,13 @@ int zn_hip_create(int device, const char *code_object_dir, zn_ctx **out) {
             std::snprintf(name, sizeof(name), "zn_attention_d%d%s", kAttnDims[d], v ? "_v" : "");
             if (hipModuleGetFunction(&ctx->attn[d][v], ctx->attn_module, name) != hipSuccess) return bail(ZN_ERR_SYMBOL);
         }
+    for (int d = 0; d < 4; ++d) {
+        char name[64];
+        std::snprintf(name, sizeof(name), "zn_attention_s%d", kAttnSplitDims[d]);
+        if (hipModuleGetFunction(&ctx->attn_split[d], ctx->attn_module, name) != hipSuccess) return bail(ZN_ERR_SYMBOL);
+    }
+    if (hipModuleGetFunction(&ctx->attn_combine, ctx->attn_module, "zn_attention_combine") != hipSuccess)
+        return bail(ZN_ERR_SYMBOL);
     void *counters = nullptr;
     if ((e = hipMalloc(&counters, kCounterSlots * kCounterStride * sizeof(int32_t))) != hipSuccess) {
         (void)hipGetLastError();
@@ -2963,19 +2976,28 @@ int zn_hip_attention_forward(zn_ctx *ctx, const float *q, const float *k, const 
     if (rc) return rc;
     const int64_t sd = seq_len * d_k, ss = seq_len * seq_len;
     if (d_k <= kAttnDims[2] && sd <= (int64_t)INT_MAX / 4 && cdiv(seq_len, kAttnQueries) <= 65535) {
-        const int dim = d_k <= kAttnDims[0] ? 0 : d_k <= kAttnDims[1] ? 1 : 2;
-        const int vec = d_k % 4 == 0 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out);
+        const int dim = (int)(d_k - 1) / 32;
         ZnAttnArgs a;
-        a.q = q;
-        a.k = k;
-        a.v = v;
-        a.out = out;
+        std::memset(&a, 0, sizeof(a));
         a.stride = sd;
         a.seq_len = (int32_t)seq_len;
         a.d_k = (int32_t)d_k;
         a.scale_log2 = scale * 1.44269504088896340736f;
         // grid.x = problem (so one problem's query blocks share an XCD), grid.y = query block
-        const int64_t gy = cdiv(seq_len, kAttnQueries);
+        const int64_t gy = cdiv(seq_len, kAttnSplitQueries[dim]);
+        // Query blocks for at most a quarter of the CUs: ranges of keys (of at
+        // least 64) for the idle ones, merged by a second launch (MI355X, one
+        // head of 1000 x 80: 159 us in 8 workgroups of the fp32 kernel, 19.6
+        // us in 8 x 16 here; 64 x 256 x 32, two ranges: 15.2 -> 22.8 us).
+        int64_t splits = std::min<int64_t>({32, cdiv(seq_len, 64), cus_now(ctx) / (batch * gy)});
+        if (splits < 4) splits = 1;
+        const int64_t keys = cdiv(cdiv(seq_len, splits), 32) * 32;
+        splits = cdiv(seq_len, keys);
+        if (splits > 1 && ensure_workspace(ctx, (size_t)(batch * seq_len * splits * (((d_k + 3) & ~3) + 4)) * sizeof(float)) != ZN_OK)
+            splits = 1;
+        a.splits = (int32_t)splits;
+        a.keys_per_split = splits > 1 ? (int32_t)keys : (int32_t)seq_len;
+        a.part = ctx->ws;
         constexpr int64_t kMaxGridX = (int64_t)1 << 30;
         for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridX) {
             const int64_t nb = batch - b0 < kMaxGridX ? batch - b0 : kMaxGridX;
@@ -2984,7 +3006,11 @@ int zn_hip_attention_forward(zn_ctx *ctx, const float *q, const float *k, const 
             c.k = k + b0 * sd;
             c.v = v + b0 * sd;
             c.out = out + b0 * sd;
-            if ((rc = launch(ctx, ctx->attn[dim][vec], (unsigned)nb, (unsigned)gy, 256, &c))) return rc;
+            c.batch = (int32_t)nb;
+            if ((rc = launch(ctx, ctx->attn_split[dim], (unsigned)nb, (unsigned)gy, kAttnSplitThreads[dim], &c, (unsigned)splits)))
+                return rc;
+            if (splits > 1 && (rc = launch(ctx, ctx->attn_combine, (unsigned)cdiv(nb * seq_len, 4), 1, 256, &c)))
+                return rc;
         }
         return ZN_OK;
     }

@@ -185,6 +185,11 @@ struct ZnAttnArgs {
     int64_t stride;
     int32_t seq_len, d_k;
     float scale_log2;  // scale * log2(e): scores are exponentiated base 2
+    // Split form with splits > 1: blockIdx.z takes keys_per_split keys (a
+    // multiple of 32) and writes its O, m and l to part, [batch * seq_len]
+    // [splits][d_k rounded up to 4, plus 4].
+    int32_t batch, splits, keys_per_split;
+    float *part;
 };
 
 // Dense backward prologue: gaa = act'(y) * grad_out elementwise and, per
