@@ -1,0 +1,167 @@
+"""GPU checks of the GEMMs on the bf16 matrix cores (zn_sgemm_<layout>_s*,
+operands split into three bf16 parts): problems of 2^30 multiply-adds and
+more with K of 256 or more, Backend.matMul and its transposes
+(src/backend.zig:169-325).
+
+- sampled rows of every layout against fp64 within 2e-7 * sqrt(K) of the
+  componentwise bound (five times tighter than the fp32 kernels' bar), at
+  extents one below and above the tiles' and at K tails of 1 to 31;
+- values near the ends of the fp32 range, where unscaled parts would be
+  subnormal, keep that bound;
+- Inf, NaN and sums beyond 2^80 give what fp32 arithmetic gives;
+- the fused epilogues, accumulation, padded leading dimensions, unaligned
+  bases and strided batches.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from _parity import uniform
+from gpu_common import announce, assert_close, ref_gemm, run_gemm, stored_shapes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from zigneuron_amd import Context
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def as_mk(a, layout):
+    return a.T if layout == "tn" else a
+
+
+def as_kn(b, layout):
+    return b.T if layout == "nt" else b
+
+
+def check_rows(out, layout, a, b, k, rows, what):
+    """Componentwise against fp64.  The bound: the flushed kernels round once per 32 of K on sums of 32, the 256x256
+    tile six times per 32 of K on the whole sum, at most 6K/32 roundings of 2^-24, which as a random walk stay under
+    sqrt(6K/32) * 2^-24 * 8 = 2e-7 * sqrt(K)."""
+    a64, b64 = as_mk(a, layout)[rows].astype(np.float64), as_kn(b, layout).astype(np.float64)
+    ref, den = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    err = np.abs(out[rows] - ref) / np.maximum(den, 1e-300)
+    assert np.isfinite(out).all() and err.max() <= 2e-7 * np.sqrt(k), f"{what}: {err.max():.3g}"
+
+
+SHAPES = [(4097, 1023, 777),    # 128x128 rows and a one-row tail
+          (4096, 1025, 257),    # one column past the tiles, K tail of 1
+          (2049, 2047, 287),    # K tail of 31
+          (4100, 4097, 288),    # a column past 32 tiles, whole K slices
+          (1025, 1023, 1027),   # 128x64 tiles
+          (300, 260, 16389),    # K in slices with the reduce
+          (8192, 131, 1030)]
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_split_against_fp64(ctx, layout, m, n, k):
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a_shape, b_shape = stored_shapes(layout, m, n, k)
+    a, b = uniform(rng, a_shape), uniform(rng, b_shape)
+    announce(f"split {layout} {m}x{n}x{k}")
+    rows = np.unique(np.r_[0, 1, m // 2, np.arange(max(0, m - 130), m, 7), m - 1])
+    check_rows(run_gemm(ctx, layout, a, b, m, n, k), layout, a, b, k, rows, f"split {layout} {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_split_largest_tile(ctx, layout):
+    """The 256x256 tile (4096 x 4096 and a K tail of 5)."""
+    m, n, k = 4095, 4096, 517
+    rng = np.random.default_rng(5)
+    a_shape, b_shape = stored_shapes(layout, m, n, k)
+    a, b = uniform(rng, a_shape), uniform(rng, b_shape)
+    announce(f"split 256x256 {layout}")
+    check_rows(run_gemm(ctx, layout, a, b, m, n, k), layout, a, b, k, np.r_[0:256:5, 3840:4095:11], "256x256")
+
+
+@pytest.mark.parametrize("scale_a,scale_b", [(2e-38, 1.0), (1.0, 2e-38), (1e-30, 1e30), (1e28, 1e-20)])
+def test_split_keeps_small_values(ctx, scale_a, scale_b):
+    """Elements at the lower end of the fp32 range (their third parts would be subnormal bf16 numbers unscaled)."""
+    m, n, k = 2049, 2047, 287
+    rng = np.random.default_rng(9)
+    a = (uniform(rng, (m, k)) * np.float32(scale_a)).astype(np.float32)
+    b = (uniform(rng, (k, n)) * np.float32(scale_b)).astype(np.float32)
+    announce(f"split range {scale_a} {scale_b}")
+    out = run_gemm(ctx, "nn", a, b, m, n, k)
+    rows = np.arange(0, m, 97)
+    a64, b64 = a[rows].astype(np.float64), b.astype(np.float64)
+    err = np.abs(out[rows] - a64 @ b64)
+    # results below 2^-126 round to multiples of 2^-149
+    assert np.all(err <= 2e-7 * np.sqrt(k) * (np.abs(a64) @ np.abs(b64)) + 2.0 ** -148)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_split_non_finite_and_huge(ctx, layout):
+    """Inf, NaN and sums past 2^80 (where the scaled split overflows): the same values as fp32 arithmetic, and the rows
+    and columns they do not touch stay within the bound."""
+    m, n, k = 2049, 2047, 287
+    rng = np.random.default_rng(10)
+    a, b = np.abs(uniform(rng, (m, k))) + np.float32(0.1), np.abs(uniform(rng, (k, n))) + np.float32(0.1)
+    a[5, 7], a[130, k - 1], a[700, 0], a[2048, 3] = np.inf, np.nan, -np.inf, np.float32(3e38)
+    a[900] *= np.float32(1e30)  # finite in fp32: 1e30 * 300
+    b[11, 40], b[2, 1000] = np.inf, np.nan
+    ast = np.ascontiguousarray(a.T) if layout == "tn" else a
+    bst = np.ascontiguousarray(b.T) if layout == "nt" else b
+    announce(f"split non-finite {layout}")
+    out = run_gemm(ctx, layout, ast, bst, m, n, k)
+    with np.errstate(all="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+        ref32 = np.where(np.abs(ref) > np.finfo(np.float32).max, np.sign(ref) * np.inf, ref)
+    fin = np.isfinite(ref32)
+    np.testing.assert_array_equal(np.isnan(out), np.isnan(ref32))
+    np.testing.assert_array_equal(np.isposinf(out), np.isposinf(ref32))
+    np.testing.assert_array_equal(np.isneginf(out), np.isneginf(ref32))
+    assert np.all(np.abs(out[fin] - ref[fin]) <= 1e-5 * np.sqrt(k) * np.abs(ref[fin]))
+
+
+@pytest.mark.parametrize("act", ["linear", "relu", "sigmoid", "tanh"])
+def test_split_epilogues(ctx, act):
+    m, n, k = 2049, 2047, 260
+    rng = np.random.default_rng(12)
+    a, b, bias = uniform(rng, (m, k)), uniform(rng, (k, n)), uniform(rng, (n,))
+    announce(f"split epilogue {act}")
+    out = run_gemm(ctx, "nn", a, b, m, n, k, bias=bias, act=act)
+    rows = np.r_[0:2049:113, 2048]
+    assert_close(out[rows], ref_gemm("nn", np.ascontiguousarray(a[rows]), b, len(rows), n, k, bias=bias, act=act), "nn",
+                 np.ascontiguousarray(a[rows]), b, len(rows), n, k, bias=bias, act=act, what=f"split {act}")
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_split_padded_rows_accumulate_batches(ctx, layout):
+    """Leading dimensions and bases off 16 bytes, accumulation, NaN in the row padding (never read as a value), and a
+    strided batch with a shared B."""
+    m, n, k, batch = 1025, 515, 273, 8
+    rng = np.random.default_rng(13)
+    a_shape, b_shape = stored_shapes(layout, m, n, k)
+    lda, ldb, ldc = a_shape[1] + 3, b_shape[1] + 1, n + 5
+    sa, sc = a_shape[0] * lda + 1, m * ldc + 3
+    a = np.full((batch, sa), np.nan, np.float32)
+    av = uniform(rng, (batch,) + a_shape)
+    a[:, :a_shape[0] * lda].reshape(batch, a_shape[0], lda)[:, :, :a_shape[1]] = av
+    b = np.full((b_shape[0], ldb), np.nan, np.float32)
+    bv = uniform(rng, b_shape)
+    b[:, :b_shape[1]] = bv
+    c0 = uniform(rng, (batch, sc))
+    da = ctx.to_device(np.concatenate([[0.0], a.ravel()]).astype(np.float32))
+    db = ctx.to_device(b)
+    dc = ctx.to_device(np.concatenate([[0.0], c0.ravel()]).astype(np.float32))
+    announce(f"split padded batch {layout}")
+    ctx.sgemm_strided_batched(layout, m, n, k, da.offset(1), lda, sa, db, ldb, 0, dc.offset(1), ldc, sc, batch, True)
+    out = dc.download()[1:].reshape(batch, sc)
+    for i in range(batch):
+        view, old = (x[i, :m * ldc].reshape(m, ldc) for x in (out, c0))
+        np.testing.assert_array_equal(view[:, n:], old[:, n:])
+        rows = np.r_[0:m:101, m - 1]
+        a64, b64 = as_mk(av[i], layout)[rows].astype(np.float64), as_kn(bv, layout).astype(np.float64)
+        ref = old[rows, :n] + a64 @ b64
+        den = np.abs(old[rows, :n]) + np.abs(a64) @ np.abs(b64)
+        assert np.all(np.abs(view[rows, :n] - ref) <= 2e-7 * np.sqrt(k) * den), i
+    np.testing.assert_array_equal(out[:, m * ldc:], c0[:, m * ldc:])
+    for buf in (da, db, dc):
+        buf.close()

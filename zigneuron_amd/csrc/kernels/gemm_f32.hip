@@ -2,6 +2,7 @@
 // intra-workgroup split-K GEMMs, the split-K reduce and the grouped Dense
 // backward launches (device code in gemm_core.h).
 #include "gemm_core.h"
+#include "gemm_split.h"
 
 // Exported kernels: zn_sgemm_<layout>_<tile>[_v].  Layout letters follow
 // the reference: nn = Backend.matMul, nt = matMulTransposeB, tn =
@@ -66,6 +67,23 @@ ZN_GEMM_R_WIDE(tn, false, false)
 ZN_GEMM_R_UNALIGNED(nn, true, false)
 ZN_GEMM_R_UNALIGNED(nt, true, true)
 ZN_GEMM_R_UNALIGNED(tn, false, false)
+// zn_sgemm_<layout>_s<tile>: operands split into bf16 parts (gemm_split.h),
+// any alignment.  sw: no flushed partial sums, whose registers would spill.
+#define ZN_GEMM_SPLIT(NAME, NW, FM, BN, AK, BKC, FLUSH, GC, AB, NV)                              \
+    extern "C" __global__ __launch_bounds__(NW * 64, 2) void NAME(ZnGemmArgs p) {                \
+        typedef SplitTile<NW, FM, BN, AK, BKC, FLUSH, GC, AB, NV> T;                             \
+        __shared__ __attribute__((aligned(1024))) char lds[2 * T::kStage];                       \
+        T::run(p, lds);                                                                          \
+    }
+#define ZN_GEMM_SPLIT_TILE(TILE, NW, FM, BN, FLUSH, GC, AB, NV)                                  \
+    ZN_GEMM_SPLIT(zn_sgemm_nn_##TILE, NW, FM, BN, true, false, FLUSH, GC, AB, NV) \
+    ZN_GEMM_SPLIT(zn_sgemm_nt_##TILE, NW, FM, BN, true, true, FLUSH, GC, AB, NV) \
+    ZN_GEMM_SPLIT(zn_sgemm_tn_##TILE, NW, FM, BN, false, false, FLUSH, GC, AB, NV)
+ZN_GEMM_SPLIT_TILE(sw, 8, 2, 256, false, 1, 1, 5)
+ZN_GEMM_SPLIT_TILE(sx, 8, 2, 128, true, 1, 2, 3)
+ZN_GEMM_SPLIT_TILE(sr, 8, 1, 128, true, 2, 2, 3)
+ZN_GEMM_SPLIT_TILE(sn, 4, 2, 64, true, 2, 2, 3)
+
 ZN_GEMM_TILE(h, gemm_tile_pinned, 64, 64, 16, 2, 2, 2)
 
 #define ZN_GEMM_WIDE(LAYOUT, AK, BKC)                                                            \

@@ -47,7 +47,10 @@ static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
 namespace {
 
 // Macro tiles of the GEMM code object (kernels/gemm_f32.hip).
-enum Tile { kTileX = 0, kTileL, kTileN, kTileM, kTileS, kTileR, kTileH, kTileW, kNumTiles };
+// The last four run on the bf16 matrix cores (three-way split operands,
+// kernels/gemm_split.h) and are chosen by size alone (choose_split).
+enum Tile { kTileX = 0, kTileL, kTileN, kTileM, kTileS, kTileR, kTileH, kTileW, kTileSW, kTileSX, kTileSR, kTileSN, kNumTiles };
+constexpr int kNumUserTiles = kTileSW;  // zn_hip_set_gemm_tile
 struct TileShape {
     int bm, bn, bk, threads;
     const char *suffix;
@@ -614,6 +617,76 @@ int choose_splits(const zn_ctx *ctx, Tile tile, int64_t m, int64_t n, int64_t k,
     return splits < 2 ? 1 : (int)splits;
 }
 
+// The split kernels (kernels/gemm_split.h, tiles sw, sx, sr and sn): each
+// operand value as three bf16 numbers, six bf16 products per fp32 product.
+struct SplitChoice {
+    Tile tile = kTileSR;
+    int splits = 1;       // K slices
+    double us = 0.0;      // estimated time
+};
+
+// Estimated time of a problem on one split tile: its workgroups on the
+// busiest CU (one resident, for sn up to two) times the time of a 32-deep
+// slice, both as measured on MI355X (us a slice: sw 4.1, sx 2.4, sr 1.5, sn
+// 1.05 alone and 1.6 two at a time), plus a round's start and stores and,
+// for K in slices, the reduce launch.
+SplitChoice estimate_split(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch, int64_t max_ws) {
+    struct Cost {
+        Tile tile;
+        double one, two;
+        bool pairs;
+    };
+    static const Cost kCosts[] = {{kTileSW, 4.1, 0, false}, {kTileSX, 2.4, 0, false}, {kTileSR, 1.5, 0, false}, {kTileSN, 1.05, 1.6, true}};
+    const int64_t cus = cus_now(ctx);
+    SplitChoice best;
+    best.us = 1e30;
+    for (const Cost &c : kCosts) {
+        const int64_t tiles = cdiv(m, kTiles[c.tile].bm) * cdiv(n, kTiles[c.tile].bn) * batch;
+        for (int64_t s = 1; s <= 16 && (s == 1 || (k / s >= 512 && 4.0 * s * batch * m * n <= (double)max_ws)); ++s) {
+            const double slices = (double)cdiv(cdiv(k, 32), s);
+            const int64_t q = cdiv(tiles * s, cus);  // workgroups on the busiest CU
+            const double rounds = c.pairs ? (double)cdiv(q, 2) : (double)q;
+            double us = 2.0 + 1.5 * rounds + slices * (c.pairs ? (q / 2) * c.two + (q % 2) * c.one : q * c.one);
+            if (s > 1) us += 3.0 + 4e-6 * (double)(s + 1) * m * n * batch / 4.0;
+            if (us < best.us) {
+                best.tile = c.tile;
+                best.splits = (int)s;
+                best.us = us;
+            }
+        }
+    }
+    return best;
+}
+
+// Rows that the split kernels take when a last row of tiles would put one
+// more workgroup on every CU: the tail rows then run as a small fp32 GEMM of
+// about 7 us (4097 x 1023 x 777: 4096 rows and one).  m when all do.
+int64_t split_main_rows(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch, SplitChoice &best) {
+    const int64_t m_main = m / 128 * 128;
+    if (batch != 1 || m_main == 0 || m_main == m || m - m_main > 32) return m;
+    SplitChoice c = estimate_split(ctx, m_main, n, k, 1, 0);
+    c.us += 7.0;
+    if (c.us >= best.us) return m;
+    best = c;
+    return m_main;
+}
+
+// Whether a problem runs on the split kernels: by its size alone, so that
+// every forced tile, every row chunk and every staging of the same problem
+// gives the same sums.  K below 256 is left to the fp32 kernels (its time is
+// mostly stores), and so is less than 2^30 multiply-adds, where one round of
+// 64x64 fp32 tiles is as fast (MI355X, 1000^3: 24.1 us split, 24.3 us fp32).
+// Above, the estimate is set against what the fp32 kernels reach: about 125
+// TFLOP/s with 128x128 tiles for most of the CUs, 95 below.
+bool split_pays(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch) {
+    const double macs = (double)m * n * k * batch;
+    if (k < 256 || macs < 1073741824.0) return false;
+    const double f32_us = 2e-6 * macs / (20 * cdiv(m, 128) * cdiv(n, 128) * batch >= 17 * cus_now(ctx) ? 125.0 : 95.0);
+    SplitChoice c = estimate_split(ctx, m, n, k, batch, (int64_t)kScratchBytes);
+    (void)split_main_rows(ctx, m, n, k, batch, c);
+    return c.us < f32_us;
+}
+
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Multiplier and shift for x / d, 0 <= x < 2^31, d >= 1: shift = ceil(log2 d),
@@ -659,11 +732,12 @@ struct RowTail {
 
 // split_rows: the launch may cut itself into two launches (a row tail; the
 // last problems of a batch), whose calls pass false.
+// arith: 0 the fp32 kernels, 1 the split kernels, -1 whichever pays.
 int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, const float *a, int64_t lda,
                    int64_t stride_a, const float *b, int64_t ldb, int64_t stride_b, float *c, int64_t ldc,
                    int64_t stride_c, int64_t batch, int accumulate, const float *bias, int act, int bias_rows,
                    const ZnConvGeom *conv = nullptr, GatherMode mode = kGatherIm2col, bool split_rows = true,
-                   int padded = 0, RowTail *row_tail = nullptr) {
+                   int padded = 0, RowTail *row_tail = nullptr, int arith = -1) {
     if (!ctx) return ZN_ERR_INVALID_ARG;
     if (layout < ZN_LAYOUT_NN || layout > ZN_LAYOUT_TN) return ZN_ERR_INVALID_ARG;
     if (act < ZN_ACT_LINEAR || act > ZN_ACT_TANH) return ZN_ERR_INVALID_ARG;
@@ -721,6 +795,26 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
                 : wn_wide                     ? kTileR
                                               : choose_tile(ctx, m, n, k, batch, conv != nullptr, native_vec);
     if (!kTiles[tile].plain && !native_vec) tile = kTileX;  // forced onto a tile it cannot stage: 256x128
+    // The split kernels, by size (forced wave splits and persistent kernels are fp32 forms)
+    const bool bf16x3 = !conv && k > 0 && ctx->forced_wave_split <= 0 && ctx->forced_persistent < 0 &&
+                        (arith == 1 || (arith < 0 && split_pays(ctx, m, n, k, batch)));
+    int policy_splits = 0;
+    if (bf16x3) {
+        // part of a larger problem: the sums of the whole, which K slices would change
+        SplitChoice ch = estimate_split(ctx, m, n, k, batch, arith == 1 ? 0 : (int64_t)kScratchBytes);
+        const int64_t m_main = split_main_rows(ctx, m, n, k, batch, ch);
+        if (split_rows && m_main < m && ctx->forced_tile < 0 && ctx->forced_splits == 0) {
+            const float *a_tail = layout == ZN_LAYOUT_TN ? a + m_main : a + m_main * lda;
+            const int rc = gemm_launch_ex(ctx, layout, m_main, n, k, a, lda, 0, b, ldb, 0, c, ldc, 0, 1, accumulate, bias, act,
+                                          bias_rows, nullptr, mode, false, padded, nullptr, 1);
+            if (rc) return rc;
+            return gemm_launch_ex(ctx, layout, m - m_main, n, k, a_tail, lda, 0, b, ldb, 0, c + m_main * ldc, ldc, 0, 1, accumulate,
+                                  bias && bias_rows ? bias + m_main : bias, act, bias_rows, nullptr, mode, false, padded,
+                                  nullptr, 0);
+        }
+        tile = ch.tile;
+        policy_splits = ch.splits;
+    }
     const TileShape &ts = kTiles[tile];
     const int64_t tiles_m = cdiv(m, ts.bm), tiles_n = cdiv(n, ts.bn);
     if (tiles_m * tiles_n > INT_MAX) return ZN_ERR_OVERFLOW;
@@ -731,7 +825,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // second, small one (usually the intra-workgroup split-K kernel).  Each
     // part is an ordinary GEMM of its rows, so no element changes its K order
     // in the first part.  Each part then makes its own staging choices.
-    if (split_rows && !conv && batch == 1 && k > 0 && ctx->forced_tile < 0 && ctx->forced_splits == 0 &&
+    if (split_rows && !conv && !bf16x3 && batch == 1 && k > 0 && ctx->forced_tile < 0 && ctx->forced_splits == 0 &&
         ctx->forced_wave_split < 0 && tiles_m >= 2) {
         const int64_t cus = cus_now(ctx);
         const int64_t ntiles_all = tiles_m * tiles_n;
@@ -742,11 +836,11 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
             // the first part may compute the tail rows too (below); if not, they are a second launch
             RowTail tail = {a_tail, c + m_main * ldc, m - m_main, false};
             int rc = gemm_launch_ex(ctx, layout, m_main, n, k, a, lda, 0, b, ldb, 0, c, ldc, 0, 1, accumulate, bias,
-                                    act, bias_rows, nullptr, mode, false, padded, &tail);
+                                    act, bias_rows, nullptr, mode, false, padded, &tail, 0);
             if (rc || tail.folded) return rc;
             return gemm_launch_ex(ctx, layout, m - m_main, n, k, a_tail, lda, 0, b, ldb, 0, c + m_main * ldc, ldc, 0, 1,
-                                  accumulate, bias_rows ? bias + m_main : bias, act, bias_rows, nullptr, mode, false,
-                                  padded);
+                                  accumulate, bias && bias_rows ? bias + m_main : bias, act, bias_rows, nullptr, mode,
+                                  false, padded, nullptr, 0);
         }
     }
     // The 128x128 register-staged tile loads rows that are not whole float4s
@@ -754,7 +848,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // takes the intra-workgroup split-K kernels below: no packed copies, no
     // 4-byte staging.
     const bool wave_split_possible =
-        !conv && k > 0 &&
+        !conv && !bf16x3 && k > 0 &&
         (ctx->forced_wave_split > 0 ||
          (ctx->forced_wave_split < 0 && ctx->forced_tile < 0 && ctx->forced_splits == 0 &&
           cdiv(m, 32) * cdiv(n, 32) * batch <= cus_now(ctx) && k >= 64 && k <= 4096));
@@ -769,7 +863,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     Lease pack_a(ctx), pack_b(ctx);
     // rows padded with zeros to whole float4s (here, or by the caller: padded bit 0 = A, bit 1 = B)
     bool a_packed = (padded & 1) != 0, b_packed = (padded & 2) != 0;
-    if (!conv && !unaligned && !ctx->no_alloc && batch == 1 && k > 0 && (double)m * n * k >= kPackMinMacs) {
+    if (!conv && !bf16x3 && !unaligned && !ctx->no_alloc && batch == 1 && k > 0 && (double)m * n * k >= kPackMinMacs) {
         const bool a_vec = aligned16(a) && lda % 4 == 0 && a_row % 4 == 0;
         const bool b_vec = aligned16(b) && ldb % 4 == 0 && b_row % 4 == 0;
         // both packings go into one launch (blockIdx.y selects the operand)
@@ -875,7 +969,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
         const int64_t wn_tiles = cdiv(m, 128) * cdiv(n, 128);
         splits = (int)std::max<int64_t>(1, std::min<int64_t>({64, cus_now(ctx) / wn_tiles, k / 768}));
     } else {
-        splits = choose_splits(ctx, tile, m, n, k, batch);
+        splits = bf16x3 ? policy_splits : choose_splits(ctx, tile, m, n, k, batch);
     }
     int64_t k_chunk = k;
     if (splits > 1) {
@@ -903,7 +997,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     args.ws = ws;
     // 4-pixel (16-byte) gather: unit column stride, and whole chunks of 4 pixels per output row
     const int gather4 = conv && conv->stride_w == 1 && conv->out_w % 4 == 0 ? 1 : 0;
-    const int staging = unaligned ? 2 : vec ? 1 : 0;  // 4-byte, 16-byte, 16-byte unaligned
+    const int staging = bf16x3 ? 0 : unaligned ? 2 : vec ? 1 : 0;  // 4-byte (split: any), 16-byte, 16-byte unaligned
     hipFunction_t f = !conv                     ? ctx->gemm[layout][tile][staging]
                       : mode == kGatherTransposed ? ctx->convt[tile][vec ? 1 : 0]
                       : mode == kGatherWeightGrad ? ctx->convw[tile][vec ? 1 : 0]
@@ -923,7 +1017,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // hand-over (stores, counter, the last workgroup's loads) costs about
     // 5 us, so below K = 1536 (C2's 256 x 128 x 784: 9.7 us unsplit, 14.1
     // split 7 ways) one workgroup per tile stays faster.
-    {
+    if (!bf16x3) {
         const int64_t cus = cus_now(ctx);
         const int64_t tiles32 = cdiv(m, 32) * cdiv(n, 32) * batch;
         int waves = 0;
@@ -1403,12 +1497,14 @@ int host_gemm_chunked(zn_ctx *ctx, int layout, const float *a, const float *b, c
             {(char *)(c + first(i) * n), (const char *)(dc + first(i) * n), count(i) * n * sizeof(float)}};
     };
     const int64_t ldb = layout == ZN_LAYOUT_NT ? (int64_t)k : (int64_t)n;
+    const int arith = split_pays(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1) ? 1 : 0;  // the whole call's, for every chunk
     if ((rc = transfer_step(ctx, ups(0), {}))) return rc;
     ZN_HIP_TRY(ctx, hipEventRecord(ctx->chunk_in[0], ctx->up));
     for (size_t i = 0; i < chunks; ++i) {
         ZN_HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, ctx->chunk_in[i & 1], 0));
-        rc = gemm_launch(ctx, layout, (int64_t)count(i), (int64_t)n, (int64_t)k, da + first(i) * k, (int64_t)k, 0,
-                         db, ldb, 0, dc + first(i) * n, (int64_t)n, 0, 1, accumulate, bias ? dbias : nullptr, act);
+        rc = gemm_launch_ex(ctx, layout, (int64_t)count(i), (int64_t)n, (int64_t)k, da + first(i) * k, (int64_t)k, 0, db,
+                            ldb, 0, dc + first(i) * n, (int64_t)n, 0, 1, accumulate, bias ? dbias : nullptr, act, 0,
+                            nullptr, kGatherIm2col, true, 0, nullptr, arith);
         if (rc) return rc;
         ZN_HIP_TRY(ctx, hipEventRecord(ctx->chunk_out[i & 1], ctx->stream));
         if (i >= 1) ZN_HIP_TRY(ctx, hipStreamWaitEvent(ctx->down, ctx->chunk_out[(i - 1) & 1], 0));
@@ -1639,7 +1735,7 @@ int zn_hip_create(int device, const char *code_object_dir, zn_ctx **out) {
     }
     for (int l = 0; l < 3; ++l)
         for (int t = 0; t < kNumTiles; ++t)
-            for (int v = kTiles[t].plain ? 0 : 1; v < (t == kTileR ? 3 : 2); ++v) {
+            for (int v = kTiles[t].plain ? 0 : 1; v < (t == kTileR ? 3 : t >= kNumUserTiles ? 1 : 2); ++v) {
                 char name[64];
                 std::snprintf(name, sizeof(name), "zn_sgemm_%s_%s%s", kLayoutName[l], kTiles[t].suffix,
                               v == 2 ? "_u" : v ? "_v" : "");
@@ -2046,7 +2142,7 @@ int zn_hip_event_destroy(zn_event *ev) {
 
 // ------------------------------------------------------------------ GEMM
 int zn_hip_set_gemm_tile(zn_ctx *ctx, int tile) {
-    if (!ctx || tile < ZN_TILE_AUTO || tile >= kNumTiles) return ZN_ERR_INVALID_ARG;
+    if (!ctx || tile < ZN_TILE_AUTO || tile >= kNumUserTiles) return ZN_ERR_INVALID_ARG;
     ctx->forced_tile = tile;
     return ZN_OK;
 }
