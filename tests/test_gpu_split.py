@@ -165,3 +165,62 @@ def test_split_padded_rows_accumulate_batches(ctx, layout):
     np.testing.assert_array_equal(out[:, m * ldc:], c0[:, m * ldc:])
     for buf in (da, db, dc):
         buf.close()
+
+
+CONVS = [(4, 64, 56, 56, 128, 3, 1, 1),   # channels a multiple of 32: one tap per K slice
+         (16, 36, 33, 35, 100, 3, 1, 1),  # taps change inside a slice; rows of 35 pixels
+         (16, 32, 61, 59, 48, 5, 2, 2),   # stride 2, 64-row tiles
+         (2, 128, 40, 40, 200, 3, 1, 0),  # no padding, 38 pixels a row
+         (33, 64, 28, 28, 64, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("case", CONVS)
+@pytest.mark.parametrize("poison", [False, True])
+def test_split_convolutions(ctx, case, poison):
+    """The convolution forward and backward (im2col branch, src/backend.zig:3881-4065) of 2^29 multiply-adds and more
+    against fp64 on the reference's im2col; poison: an Inf in the input and a NaN in grad_output reach exactly the
+    results they reach in fp64."""
+    from oracle import oracle
+    B, C, H, W, OC, ker, st, pd = case
+    OH, OW = (H + 2 * pd - ker) // st + 1, (W + 2 * pd - ker) // st + 1
+    rng = np.random.default_rng(sum(case))
+    x, w = uniform(rng, (B, C, H, W)), uniform(rng, (OC, ker * ker * C))
+    bias, g = uniform(rng, (OC,)), uniform(rng, (B * OH * OW, OC))
+    if poison:
+        x[B - 1, 3, H // 2, W - 1] = np.inf
+        g[7, 2] = np.nan
+    dx, dw, db, dg = (ctx.to_device(a) for a in (x, w, bias, g))
+    y, gx, gw, gb = (ctx.alloc(n).fill(0.5) for n in (B * OC * OH * OW, x.size, w.size, OC))
+    geom = (B, C, OC, ker, ker, H, W, OH, OW, st, st, pd, pd)
+    announce(f"split convolution {case} poison {poison}")
+    ctx.conv2d_forward_im2col(dx, dw, db, y, *geom)
+    ctx.conv2d_backward_im2col(dx, dw, dg, gx, gw, gb, *geom)
+    col = oracle.im2col(x, B, C, H, W, ker, ker, stride=(st, st), pad=(pd, pd)).reshape(B * OH * OW, -1).astype(np.float64)
+    w64, g64 = w.astype(np.float64), g.astype(np.float64)
+
+    def check(got, ref, den, k, what):
+        fin = np.isfinite(ref)
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(ref), err_msg=what)
+        np.testing.assert_array_equal(np.isinf(got), np.isinf(ref), err_msg=what)
+        assert np.all(np.abs(got[fin] - ref[fin]) <= (1e-5 if poison else 4e-7) * np.sqrt(k) * den[fin]), what
+
+    with np.errstate(all="ignore"):
+        taps = ker * ker * C
+        ref = col @ w64.T + bias
+        den = np.where(np.isfinite(ref), np.nan_to_num(np.abs(col), posinf=0) @ np.abs(w64).T + np.abs(bias), 0)
+        check(y.download().reshape(B, OC, OH * OW).transpose(0, 2, 1).reshape(-1, OC), ref, den, taps, "forward")
+        ref = g64.T @ col
+        den = np.nan_to_num(np.abs(g64)).T @ np.nan_to_num(np.abs(col), posinf=0)
+        check(gw.download().reshape(OC, taps), ref, den, B * OH * OW, "weight gradient")
+        gcol, dcol = g64 @ w64, np.nan_to_num(np.abs(g64)) @ np.abs(w64)
+        ref, den = (np.zeros((B, H + 2 * pd, W + 2 * pd, C)) for _ in range(2))
+        for kh in range(ker):
+            for kw in range(ker):
+                at = np.s_[:, kh:kh + st * OH:st, kw:kw + st * OW:st]
+                sl = np.s_[:, (kh * ker + kw) * C:(kh * ker + kw + 1) * C]
+                ref[at] += gcol[sl].reshape(B, OH, OW, C)
+                den[at] += dcol[sl].reshape(B, OH, OW, C)
+        inner = np.s_[:, pd:pd + H, pd:pd + W]
+        check(gx.download().reshape(B, C, H, W).transpose(0, 2, 3, 1), ref[inner], den[inner], taps // C * OC, "input gradient")
+    for b in (dx, dw, db, dg, y, gx, gw, gb):
+        b.close()

@@ -8,6 +8,7 @@
 // K granularity for the 64x64 tile (32: split-K chunks, the NHWC forward's
 // one-tap slices) is a multiple of that BK.
 #include "gemm_core.h"
+#include "gemm_split.h"
 
 // Implicit-GEMM convolution, per image b = blockIdx.y:
 // out_b[OC][OH*OW] = W[OC][K] . im2col(input_b)^T (+ bias[oc]), an NN GEMM
@@ -107,3 +108,19 @@ extern "C" __global__ __launch_bounds__(512, 1) void zn_convwn_tn_r_v(ZnGemmArgs
     gemm_tile_wide<128, 128, 16, 2, 4, false, false, kGNhwcW>(p);
 }
 ZN_CONVWN_TILE(s, gemm_tile_dma, 32, 32, 32, 1, 1, 1)
+
+// The NHWC forward, the transposed convolution and the NHWC weight gradient
+// on the bf16 matrix cores (gemm_split.h): 128x128 tiles (cr), and 64x128
+// ones (ch) for few output rows.
+#define ZN_CONV_SPLIT(NAME, NW, AK, BKC, G, MINB)                                                \
+    extern "C" __global__ __launch_bounds__(NW * 64, MINB) void NAME(ZnGemmArgs p) {             \
+        typedef SplitTile<NW, 1, 128, AK, BKC, true, 2, 2, 3, G> T;                              \
+        __shared__ __attribute__((aligned(1024))) char lds[2 * T::kStage];                       \
+        T::run(p, lds);                                                                          \
+    }
+ZN_CONV_SPLIT(zn_convfs_nt_cr, 8, true, true, kGNhwc, 2)
+ZN_CONV_SPLIT(zn_convfs_nt_ch, 4, true, true, kGNhwc, 2)
+ZN_CONV_SPLIT(zn_convts_nt_cr, 8, true, true, kGTransposed, 2)
+ZN_CONV_SPLIT(zn_convts_nt_ch, 4, true, true, kGTransposed, 2)
+ZN_CONV_SPLIT(zn_convwns_tn_cr, 8, false, false, kGNhwcW, 2)
+ZN_CONV_SPLIT(zn_convwns_tn_ch, 4, false, false, kGNhwcW, 2)

@@ -41,7 +41,7 @@ namespace {
 //    nothing.
 //  * Sums that are not finite: the wave does its tile again on the fp32
 //    matrix cores (plain), about five times slower.
-template <int NW, int FM, int BN, bool AK, bool BKC, bool FLUSH, int GC, int AB, int NV>
+template <int NW, int FM, int BN, bool AK, bool BKC, bool FLUSH, int GC, int AB, int NV, int G = kGNone>
 struct SplitTile {
     static constexpr int NT = NW * kWave;
     static constexpr int BM = 16 * FM * NW, BK = 32;
@@ -51,6 +51,11 @@ struct SplitTile {
     static constexpr int kPartB = BN * kRowBytes;
     static constexpr int kStage = 3 * kPartB;
     static_assert(BN * 4 % NT == 0 && BN % kWave == 0, "whole units per thread; a wave's X-contiguous loads share one k");
+
+    static constexpr bool GATHER_K = G == kGNhwc || G == kGTransposed;  // convolutions: B gathered K-contiguously
+    static constexpr bool GATHER_X = G == kGNhwcW;                      // ... or X-contiguously
+    static_assert(G == kGNone || (GATHER_K && BKC) || (GATHER_X && !BKC), "the NHWC gathers");
+    static constexpr int kNoRow = -(1 << 30);  // an image row that no tap reaches
 
     // slot of chunk c (8 k, 16 bytes) of LDS row r: the chunks of 4 rows fill the 64 banks, and the rotation spreads the
     // 16 rows of each of the hardware's four 16-lane groups of a ds_read_b128 (lanes 0-3, 12-15, 20-27; ...) over them
@@ -84,7 +89,12 @@ struct SplitTile {
         const int ktiles = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
         const int lda = (int)p.lda, ldb = (int)p.ldb;
         const uint32_t a_bytes = (uint32_t)(AK ? (p.m - 1) * lda + p.k : (p.k - 1) * lda + p.m) * 4u;
-        const uint32_t b_bytes = (uint32_t)(BKC ? (p.n - 1) * ldb + p.k : (p.k - 1) * ldb + p.n) * 4u;
+        const ZnConvGeom &cg = p.conv;
+        const uint32_t b_bytes =
+            (uint32_t)(GATHER_K   ? cg.channels * cg.in_h * cg.in_w
+                       : GATHER_X ? cg.images * cg.channels * cg.in_h * cg.in_w
+                       : BKC      ? (p.n - 1) * ldb + p.k
+                                  : (p.k - 1) * ldb + p.n) * 4u;
         const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a + bz * p.stride_a, a_bytes);
         const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.b + bz * p.stride_b, b_bytes);
 
@@ -92,6 +102,7 @@ struct SplitTile {
         // A: this lane's rows 16f + li, chunk lh.  B: staging units (row, chunk).
         uint32_t offa[FM], offb[UB];
         int lpos[UB], kq[UB];
+        int gh[UB], gw[UB];  // gathers: image row and column of the unit's pixel (K) or tap (X), before the other's share
 #pragma unroll
         for (int f = 0; f < FM; ++f) {
             const int x = m0 + 16 * f + li;
@@ -105,6 +116,18 @@ struct SplitTile {
             kq[j] = BKC ? 4 * c : __builtin_amdgcn_readfirstlane(4 * c);
             offb[j] = x < p.n ? (uint32_t)(BKC ? x * ldb + kbeg + 4 * c : x) * 4u : kOutOfRange;
             lpos[j] = slot(row, c);
+            if constexpr (GATHER_K) {
+                const int oh = zn_udiv(x, cg.ow_mul, cg.ow_shift), ow = x - oh * cg.out_w;
+                gh[j] = x >= p.n ? kNoRow : G == kGNhwc ? oh * cg.stride_h - cg.pad_h : oh + cg.pad_h;
+                gw[j] = G == kGNhwc ? ow * cg.stride_w - cg.pad_w : ow + cg.pad_w;
+            }
+            if constexpr (GATHER_X) {
+                const int khw = zn_udiv(x, cg.div1_mul, cg.div1_shift), ic = x - khw * cg.div1;
+                const int kh = zn_udiv(khw, cg.kw_mul, cg.kw_shift), kw = khw - kh * cg.k_w;
+                gh[j] = x < p.n ? kh - cg.pad_h : kNoRow;
+                gw[j] = kw - cg.pad_w;
+                offb[j] = (uint32_t)(((kh - cg.pad_h) * cg.in_w + gw[j]) * cg.channels + ic) * 4u;
+            }
         }
         float ga[FM][8], gb[UB][8];  // the raw values of the next slice
         auto load_k = [&](__amdgpu_buffer_rsrc_t r, uint32_t off0, int s, float(&g)[8]) {
@@ -139,8 +162,77 @@ struct SplitTile {
                 }
             }
         };
+        // byte offset of channel ic under tap (kh, kw) of unit j's pixel, or out of range in the padding
+        auto gather_k = [&](int j, int kh, int kw, int ic) {
+            const int ih = G == kGNhwc ? gh[j] + kh : gh[j] - kh, iw = G == kGNhwc ? gw[j] + kw : gw[j] - kw;
+            const bool ok = (unsigned)ih < (unsigned)cg.in_h && (unsigned)iw < (unsigned)cg.in_w;
+            return ok ? (uint32_t)((ih * cg.in_w + iw) * cg.channels + ic) * 4u : kOutOfRange;
+        };
         auto load_b = [&](int s, int j, float(&g)[8]) {
-            if constexpr (BKC) {
+            if constexpr (GATHER_K) {
+                // 4 consecutive channels of one tap a load (channels are a multiple of 4); tap_uniform: the whole slice
+                // lies in one tap, decoded on the scalar unit
+                const int k0 = kbeg + s * BK;
+                uint32_t off[2];
+                if (cg.tap_uniform) {
+                    const int khw = zn_udiv(k0, cg.div1_mul, cg.div1_shift);
+                    const int kh = zn_udiv(khw, cg.kw_mul, cg.kw_shift);
+                    off[0] = gather_k(j, kh, khw - kh * cg.k_w, k0 - khw * cg.div1 + kq[j]);
+                    off[1] = off[0] + 64;
+                } else {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int k = k0 + kq[j] + 16 * h;
+                        const int khw = zn_udiv(k, cg.div1_mul, cg.div1_shift);
+                        const int kh = zn_udiv(khw, cg.kw_mul, cg.kw_shift);
+                        off[h] = k < kend ? gather_k(j, kh, khw - kh * cg.k_w, k - khw * cg.div1) : kOutOfRange;
+                    }
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const zn_f32x4 v = __builtin_bit_cast(zn_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, off[h], 0, 0));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) g[4 * h + e] = v[e];
+                }
+            } else if constexpr (GATHER_X) {
+                // 64 channels-under-a-tap of one output pixel a load; the pixel is wave-uniform.  Rows of whole quads of
+                // pixels: one decode for each 4 consecutive pixels.
+                const int plane = cg.channels * cg.in_h * cg.in_w;
+                uint32_t off[8];
+                auto pixel = [&](int k, int &base, int &oh, int &ow) {
+                    k = min(k, kend - 1);  // pixels past the end meet zeros of A
+                    const int q = zn_udiv(k, cg.ow_mul, cg.ow_shift);
+                    const int b = zn_udiv(q, cg.oh_mul, cg.oh_shift);
+                    ow = (k - q * cg.out_w) * cg.stride_w;
+                    oh = (q - b * cg.out_h) * cg.stride_h;
+                    base = b * plane + (oh * cg.in_w + ow) * cg.channels;
+                };
+                auto place = [&](int base, int oh, int ow) {
+                    const bool ok = (unsigned)(gh[j] + oh) < (unsigned)cg.in_h && (unsigned)(gw[j] + ow) < (unsigned)cg.in_w;
+                    return ok ? offb[j] + (uint32_t)base * 4u : kOutOfRange;
+                };
+                const int k0 = kbeg + s * BK + kq[j];
+                if (cg.out_w % 4 == 0) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        int base, oh, ow;
+                        pixel(k0 + 16 * h, base, oh, ow);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            off[4 * h + e] = place(base + e * cg.stride_w * cg.channels, oh, ow + e * cg.stride_w);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        int base, oh, ow;
+                        pixel(k0 + (e < 4 ? e : 12 + e), base, oh, ow);
+                        off[e] = place(base, oh, ow);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    g[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, off[e], 0, 0));
+            } else if constexpr (BKC) {
                 load_k(rb, offb[j], s, g);
             } else {
                 const int k0 = kbeg + s * BK + kq[j];
@@ -306,7 +398,19 @@ struct SplitTile {
 #pragma unroll
             for (int f = 0; f < FN; ++f) {
                 const int x = nw + 16 * f + li;
-                const uint32_t off = x < p.n && kk < kend ? (uint32_t)(BKC ? x * ldb + kk : kk * ldb + x) * 4u : kOutOfRange;
+                uint32_t off = x < p.n && kk < kend ? (uint32_t)(BKC ? x * ldb + kk : kk * ldb + x) * 4u : kOutOfRange;
+                if constexpr (G != kGNone) {
+                    const ZnConvGeom &cg = p.conv;
+                    const int px = GATHER_X ? kk : x, tap = GATHER_X ? x : kk;
+                    const int khw = zn_udiv(tap, cg.div1_mul, cg.div1_shift), ic = tap - khw * cg.div1;
+                    const int kh = zn_udiv(khw, cg.kw_mul, cg.kw_shift), kw = khw - kh * cg.k_w;
+                    const int q = zn_udiv(px, cg.ow_mul, cg.ow_shift), ow = px - q * cg.out_w;
+                    const int img = GATHER_X ? zn_udiv(q, cg.oh_mul, cg.oh_shift) : 0, oh = q - img * cg.out_h;
+                    const int ih = G == kGTransposed ? q + cg.pad_h - kh : (GATHER_X ? oh : q) * cg.stride_h - cg.pad_h + kh;
+                    const int iw = G == kGTransposed ? ow + cg.pad_w - kw : ow * cg.stride_w - cg.pad_w + kw;
+                    const bool ok = off != kOutOfRange && (unsigned)ih < (unsigned)cg.in_h && (unsigned)iw < (unsigned)cg.in_w;
+                    off = ok ? (uint32_t)(((img * cg.in_h + ih) * cg.in_w + iw) * cg.channels + ic) * 4u : kOutOfRange;
+                }
                 b[f] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, off, 0, 0));
             }
 #pragma unroll

@@ -47,9 +47,10 @@ static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
 namespace {
 
 // Macro tiles of the GEMM code object (kernels/gemm_f32.hip).
-// The last four run on the bf16 matrix cores (three-way split operands,
-// kernels/gemm_split.h) and are chosen by size alone (choose_split).
-enum Tile { kTileX = 0, kTileL, kTileN, kTileM, kTileS, kTileR, kTileH, kTileW, kTileSW, kTileSX, kTileSR, kTileSN, kNumTiles };
+// The last six run on the bf16 matrix cores (three-way split operands,
+// kernels/gemm_split.h) and are chosen by size alone (split_pays); cr and ch
+// are the convolutions'.
+enum Tile { kTileX = 0, kTileL, kTileN, kTileM, kTileS, kTileR, kTileH, kTileW, kTileSW, kTileSX, kTileSR, kTileSN, kTileCR, kTileCH, kNumTiles };
 constexpr int kNumUserTiles = kTileSW;  // zn_hip_set_gemm_tile
 struct TileShape {
     int bm, bn, bk, threads;
@@ -69,7 +70,9 @@ constexpr TileShape kTiles[kNumTiles] = {{256, 128, 16, 512, "x", true, true, tr
                                          {256, 256, 32, 512, "sw", false, false, true},
                                          {256, 128, 32, 512, "sx", false, false, true},
                                          {128, 128, 32, 512, "sr", false, false, true},
-                                         {128, 64, 32, 256, "sn", false, false, true}};
+                                         {128, 64, 32, 256, "sn", false, false, true},
+                                         {128, 128, 32, 512, "cr", false, false, false},
+                                         {64, 128, 32, 256, "ch", false, false, false}};
 constexpr const char *kLayoutName[3] = {"nn", "nt", "tn"};
 
 enum EltKernel { kFill, kCopy, kAddBias, kActFwd, kActBwd, kAccBias, kIm2col, kSoftmax, kCol2im, kRowSum, kDenseGrad, kRegroup, kPack, kToNhwc, kHold, kCol2imPx, kNumElt };
@@ -187,6 +190,7 @@ struct zn_ctx {
     hipFunction_t dense_bwd_k[2] = {};         // the same on 32x32 tiles with K split over 4 waves [16-byte]
     hipFunction_t convf[kNumTiles][2] = {};    // convolution forward on NHWC [tile][16-byte W rows]
     hipFunction_t convwn[kNumTiles][2] = {};   // weight gradient on NHWC [tile][16-byte grad_output rows]
+    hipFunction_t conv_split[3][2] = {};       // [forward, input, weight gradient][cr, ch]: the bf16 matrix cores
     hipFunction_t gemmp[3][kNumTiles] = {};    // persistent plain GEMM, 16-byte staging [layout][tile] (not s)
     hipFunction_t gemmk[3][2][2] = {};         // intra-workgroup split-K, 32x32 tiles [layout][4 or 8 waves][16-byte]
     int gemmp_occ[3][kNumTiles] = {};          // its resident workgroups per CU
@@ -647,7 +651,7 @@ SplitChoice estimate_split(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, i
             const int64_t q = cdiv(tiles * s, cus);  // workgroups on the busiest CU
             const double rounds = c.pairs ? (double)cdiv(q, 2) : (double)q;
             double us = 2.0 + 1.5 * rounds + slices * (c.pairs ? (q / 2) * c.two + (q % 2) * c.one : q * c.one);
-            if (s > 1) us += 3.0 + 4e-6 * (double)(s + 1) * m * n * batch / 4.0;
+            if (s > 1) us += 4.0 + 4e-6 * (double)(s + 1) * m * n * batch / 1.8;  // the partial sums, 1.8 TB/s
             if (us < best.us) {
                 best.tile = c.tile;
                 best.splits = (int)s;
@@ -685,6 +689,28 @@ bool split_pays(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batc
     SplitChoice c = estimate_split(ctx, m, n, k, batch, (int64_t)kScratchBytes);
     (void)split_main_rows(ctx, m, n, k, batch, c);
     return c.us < f32_us;
+}
+
+// The tile a gathered convolution GEMM (M rows, N columns, `batch` images)
+// takes on the split kernels, or kNumTiles when the fp32 kernels are kept:
+// less than 2^29 multiply-adds, K below 128, fewer than 33 rows (half the
+// tile padding), or an estimate above the 95 TFLOP/s those reach.  Measured
+// us a slice, one workgroup a CU: cr 1.5, ch 1.0.
+Tile conv_split_tile(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch, int64_t splits) {
+    const double macs = (double)m * n * k * batch;
+    if (k < 128 || m < 33 || macs < 536870912.0) return kNumTiles;
+    Tile best = kNumTiles;
+    double best_us = 2e-6 * macs / 95.0;
+    for (Tile t : {kTileCR, kTileCH}) {
+        const int64_t tiles = cdiv(m, kTiles[t].bm) * cdiv(n, kTiles[t].bn) * batch * splits;
+        const double per = t == kTileCR ? 1.5 : 1.0, q = (double)cdiv(tiles, cus_now(ctx));
+        const double us = 2.0 + q * (1.5 + per * (double)cdiv(cdiv(k, 32), splits));
+        if (us < best_us) {
+            best = t;
+            best_us = us;
+        }
+    }
+    return best;
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -799,6 +825,23 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     const bool bf16x3 = !conv && k > 0 && ctx->forced_wave_split <= 0 && ctx->forced_persistent < 0 &&
                         (arith == 1 || (arith < 0 && split_pays(ctx, m, n, k, batch)));
     int policy_splits = 0;
+    const bool conv_policy = conv && !forced && ctx->forced_splits == 0 && ctx->forced_persistent < 0 && k > 0;
+    bool conv_split = false;
+    if (conv_policy && (mode == kGatherNhwc || mode == kGatherTransposed)) {
+        const Tile t = conv_split_tile(ctx, m, n, k, batch, 1);
+        if ((conv_split = t != kNumTiles)) {
+            tile = t;
+            policy_splits = 1;
+        }
+    } else if (conv_policy && mode == kGatherWeightNhwc && k >= 64 * 128) {
+        // few tiles over every output pixel: K slices for one round of workgroups
+        const int64_t tiles = cdiv(m, 128) * cdiv(n, 128);
+        const int64_t s = std::max<int64_t>(1, std::min<int64_t>({64, cus_now(ctx) / tiles, k / 768}));
+        if ((conv_split = conv_split_tile(ctx, m, n, k, 1, s) != kNumTiles)) {
+            tile = m > 64 ? kTileCR : kTileCH;
+            policy_splits = (int)std::max<int64_t>(1, std::min<int64_t>({64, cus_now(ctx) / (cdiv(m, kTiles[tile].bm) * cdiv(n, 128)), k / 768}));
+        }
+    }
     if (bf16x3) {
         // part of a larger problem: the sums of the whole, which K slices would change
         SplitChoice ch = estimate_split(ctx, m, n, k, batch, arith == 1 ? 0 : (int64_t)kScratchBytes);
@@ -923,7 +966,8 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     args.bias_rows = bias_rows ? 1 : 0;
     if (conv) args.conv = *conv;
     // NHWC forward: each BK slice of K lies in one filter tap when the channels are whole slices
-    if (conv && mode == kGatherNhwc) args.conv.tap_uniform = conv->channels % ts.bk == 0 ? 1 : 0;
+    if (conv && (mode == kGatherNhwc || (conv_split && mode == kGatherTransposed)))
+        args.conv.tap_uniform = conv->channels % ts.bk == 0 ? 1 : 0;
     // 16-byte staging: aligned rows and contiguous extents that are whole float4s
     const bool vec = conv ? (aligned16(a) && lda % 4 == 0 && stride_a % 4 == 0 && a_row % 4 == 0)
                           : (aligned16(a) && aligned16(b) && lda % 4 == 0 && ldb % 4 == 0 && stride_a % 4 == 0 &&
@@ -943,7 +987,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // (MI355X, C5's 49 tiles per image on 1536 resident workgroups: 147.8 us
     // for 31 images, 168.8 us for 32).  The last problems go to a launch of
     // their own, which the split-K policy spreads over every CU.
-    if (conv && mode == kGatherTransposed && split_rows && batch > 1 && !forced && ctx->forced_splits == 0) {
+    if (conv && mode == kGatherTransposed && !conv_split && split_rows && batch > 1 && !forced && ctx->forced_splits == 0) {
         const int64_t slots = cus_now(ctx) * ctx->convt_occ[tile][vec ? 1 : 0];
         const int64_t total = ntiles * batch, rem = total % slots;
         const int64_t r = cdiv(rem, ntiles);  // problems holding the last round's tiles
@@ -965,11 +1009,11 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     int splits;
     if (ctx->forced_splits > 0) {
         splits = (int)std::min<int64_t>(ctx->forced_splits, std::max<int64_t>(1, cdiv(k, ts.bk)));
-    } else if (wn_wide && !forced) {  // one round: CUs / tiles slices, at most 64, at least 768 of K each
+    } else if (wn_wide && !forced && !conv_split) {  // one round: CUs / tiles slices, at most 64, at least 768 of K each
         const int64_t wn_tiles = cdiv(m, 128) * cdiv(n, 128);
         splits = (int)std::max<int64_t>(1, std::min<int64_t>({64, cus_now(ctx) / wn_tiles, k / 768}));
     } else {
-        splits = bf16x3 ? policy_splits : choose_splits(ctx, tile, m, n, k, batch);
+        splits = bf16x3 || conv_split ? policy_splits : choose_splits(ctx, tile, m, n, k, batch);
     }
     int64_t k_chunk = k;
     if (splits > 1) {
@@ -998,7 +1042,8 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // 4-pixel (16-byte) gather: unit column stride, and whole chunks of 4 pixels per output row
     const int gather4 = conv && conv->stride_w == 1 && conv->out_w % 4 == 0 ? 1 : 0;
     const int staging = bf16x3 ? 0 : unaligned ? 2 : vec ? 1 : 0;  // 4-byte (split: any), 16-byte, 16-byte unaligned
-    hipFunction_t f = !conv                     ? ctx->gemm[layout][tile][staging]
+    hipFunction_t f = conv_split ? ctx->conv_split[mode == kGatherNhwc ? 0 : mode == kGatherTransposed ? 1 : 2][tile - kTileCR]
+                      : !conv                     ? ctx->gemm[layout][tile][staging]
                       : mode == kGatherTransposed ? ctx->convt[tile][vec ? 1 : 0]
                       : mode == kGatherWeightGrad ? ctx->convw[tile][vec ? 1 : 0]
                       : mode == kGatherNhwc       ? ctx->convf[tile][vec ? 1 : 0]
@@ -1146,6 +1191,10 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
         ZnGemmArgs part = args;
         part.batch = (int32_t)nb;
         if (splits > 1 && nb == 1) part.xcd_remap = 2;  // the tiles of one K slice share an XCD's L2
+        // split 128-row tiles: each XCD a contiguous run of them, which share
+        // A panels (4096 x 1024 x 1024 NN 50.1 -> 48.9 us, NT 48.2 -> 46.9)
+        else if (bf16x3 && splits == 1 && nb == 1 && (tile == kTileSR || tile == kTileSN) && ntiles % 8 == 0)
+            part.xcd_remap = 1;
         part.a = a ? a + b0 * stride_a : nullptr;
         part.b = b ? b + b0 * stride_b : nullptr;
         part.c = c + b0 * stride_c;
@@ -1735,7 +1784,7 @@ int zn_hip_create(int device, const char *code_object_dir, zn_ctx **out) {
     }
     for (int l = 0; l < 3; ++l)
         for (int t = 0; t < kNumTiles; ++t)
-            for (int v = kTiles[t].plain ? 0 : 1; v < (t == kTileR ? 3 : t >= kNumUserTiles ? 1 : 2); ++v) {
+            for (int v = kTiles[t].plain ? 0 : 1; t < kTileCR && v < (t == kTileR ? 3 : t >= kNumUserTiles ? 1 : 2); ++v) {
                 char name[64];
                 std::snprintf(name, sizeof(name), "zn_sgemm_%s_%s%s", kLayoutName[l], kTiles[t].suffix,
                               v == 2 ? "_u" : v ? "_v" : "");
@@ -1781,6 +1830,14 @@ int zn_hip_create(int device, const char *code_object_dir, zn_ctx **out) {
     // the 128x128 tile's only convolution kernel: the NHWC weight gradient, 16-byte rows
     if (hipModuleGetFunction(&ctx->convwn[kTileR][1], ctx->conv_module, "zn_convwn_tn_r_v") != hipSuccess)
         return bail(ZN_ERR_SYMBOL);
+    for (int g = 0; g < 3; ++g)
+        for (int t = 0; t < 2; ++t) {
+            static const char *kFamily[3] = {"zn_convfs_nt", "zn_convts_nt", "zn_convwns_tn"};
+            char name[64];
+            std::snprintf(name, sizeof(name), "%s_%s", kFamily[g], kTiles[kTileCR + t].suffix);
+            if (hipModuleGetFunction(&ctx->conv_split[g][t], ctx->conv_module, name) != hipSuccess)
+                return bail(ZN_ERR_SYMBOL);
+        }
     for (int l = 0; l < 3; ++l)
         for (int w = 0; w < 2; ++w)
             for (int v = 0; v < 2; ++v) {
@@ -3071,7 +3128,32 @@ int zn_hip_attention_forward(zn_ctx *ctx, const float *q, const float *k, const 
     int rc = select_device(ctx);
     if (rc) return rc;
     const int64_t sd = seq_len * d_k, ss = seq_len * seq_len;
-    if (d_k <= kAttnDims[2] && sd <= (int64_t)INT_MAX / 4 && cdiv(seq_len, kAttnQueries) <= 65535) {
+    // Short sequences of narrow heads stay on the fp32 kernels, whose smaller
+    // workgroups start sooner (MI355X: 128 x 128 x 64 13.6 us, split 17.0; 32
+    // x 192 x 64 17.3 and 22.7; 64 x 256 x 32 13.0 and 13.4; from 512 on the
+    // split form is 1.5 times as fast, and above 64 head dims always faster).
+    if (d_k <= kAttnDims[1] && seq_len <= 256) {
+        const int dim = d_k <= kAttnDims[0] ? 0 : 1;
+        const int vec = d_k % 4 == 0 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out);
+        ZnAttnArgs a;
+        std::memset(&a, 0, sizeof(a));
+        a.stride = sd;
+        a.seq_len = (int32_t)seq_len;
+        a.d_k = (int32_t)d_k;
+        a.scale_log2 = scale * 1.44269504088896340736f;
+        constexpr int64_t kMaxGridX = (int64_t)1 << 30;
+        for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridX) {
+            const int64_t nb = batch - b0 < kMaxGridX ? batch - b0 : kMaxGridX;
+            ZnAttnArgs c = a;
+            c.q = q + b0 * sd;
+            c.k = k + b0 * sd;
+            c.v = v + b0 * sd;
+            c.out = out + b0 * sd;
+            if ((rc = launch(ctx, ctx->attn[dim][vec], (unsigned)nb, (unsigned)cdiv(seq_len, kAttnQueries), 256, &c))) return rc;
+        }
+        return ZN_OK;
+    }
+    if (d_k <= kAttnSplitDims[3] && sd <= (int64_t)INT_MAX / 4 && cdiv(seq_len, kAttnQueries) <= 65535) {
         const int dim = (int)(d_k - 1) / 32;
         ZnAttnArgs a;
         std::memset(&a, 0, sizeof(a));
