@@ -171,7 +171,8 @@ CONVS = [(4, 64, 56, 56, 128, 3, 1, 1),   # channels a multiple of 32: one tap p
          (16, 36, 33, 35, 100, 3, 1, 1),  # taps change inside a slice; rows of 35 pixels
          (16, 32, 61, 59, 48, 5, 2, 2),   # stride 2, 64-row tiles
          (2, 128, 40, 40, 200, 3, 1, 0),  # no padding, 38 pixels a row
-         (33, 64, 28, 28, 64, 3, 1, 1)]
+         (33, 64, 28, 28, 64, 3, 1, 1),
+         (16, 32, 63, 63, 128, 3, 2, 1)]  # stride 2 with whole fours of pixels a row
 
 
 @pytest.mark.parametrize("case", CONVS)

@@ -111,16 +111,25 @@ ZN_CONVWN_TILE(s, gemm_tile_dma, 32, 32, 32, 1, 1, 1)
 
 // The NHWC forward, the transposed convolution and the NHWC weight gradient
 // on the bf16 matrix cores (gemm_split.h): 128x128 tiles (cr), and 64x128
-// ones (ch) for few output rows.
-#define ZN_CONV_SPLIT(NAME, NW, AK, BKC, G, MINB)                                                \
+// ones (ch) for few output rows; _u: one decode of the gather for each slice
+// of K (the filter tap) or 4 of it (the output row), and no branch inside a
+// step (C5's weight gradient GEMM 140 -> 128 us: 315 scalar instructions a
+// slice before, 80 now).  cr of the forward and the input gradient: one
+// column block at a time fits 128 registers, two workgroups to a CU (C5's
+// forward GEMM 123 -> 106 us); the weight gradient, one round of workgroups,
+// would spill there (217 us), and ch measured the same with either.
+#define ZN_CONV_SPLIT(NAME, NW, AK, BKC, G, GU, GC, MINB)                                        \
     extern "C" __global__ __launch_bounds__(NW * 64, MINB) void NAME(ZnGemmArgs p) {             \
-        typedef SplitTile<NW, 1, 128, AK, BKC, true, 2, 2, 3, G> T;                              \
+        typedef SplitTile<NW, 1, 128, AK, BKC, true, GC, 2, 3, G, GU> T;                         \
         __shared__ __attribute__((aligned(1024))) char lds[2 * T::kStage];                       \
         T::run(p, lds);                                                                          \
     }
-ZN_CONV_SPLIT(zn_convfs_nt_cr, 8, true, true, kGNhwc, 2)
-ZN_CONV_SPLIT(zn_convfs_nt_ch, 4, true, true, kGNhwc, 2)
-ZN_CONV_SPLIT(zn_convts_nt_cr, 8, true, true, kGTransposed, 2)
-ZN_CONV_SPLIT(zn_convts_nt_ch, 4, true, true, kGTransposed, 2)
-ZN_CONV_SPLIT(zn_convwns_tn_cr, 8, false, false, kGNhwcW, 2)
-ZN_CONV_SPLIT(zn_convwns_tn_ch, 4, false, false, kGNhwcW, 2)
+#define ZN_CONV_SPLIT_TILE(TILE, NW, GC, MINB, WGC, WMINB)                                       \
+    ZN_CONV_SPLIT(zn_convfs_nt_##TILE, NW, true, true, kGNhwc, false, GC, MINB)                  \
+    ZN_CONV_SPLIT(zn_convfs_nt_##TILE##_u, NW, true, true, kGNhwc, true, GC, MINB)               \
+    ZN_CONV_SPLIT(zn_convts_nt_##TILE, NW, true, true, kGTransposed, false, GC, MINB)            \
+    ZN_CONV_SPLIT(zn_convts_nt_##TILE##_u, NW, true, true, kGTransposed, true, GC, MINB)         \
+    ZN_CONV_SPLIT(zn_convwns_tn_##TILE, NW, false, false, kGNhwcW, false, WGC, WMINB)            \
+    ZN_CONV_SPLIT(zn_convwns_tn_##TILE##_u, NW, false, false, kGNhwcW, true, WGC, WMINB)
+ZN_CONV_SPLIT_TILE(cr, 8, 1, 4, 2, 2)
+ZN_CONV_SPLIT_TILE(ch, 4, 2, 2, 2, 2)

@@ -41,7 +41,7 @@ namespace {
 //    nothing.
 //  * Sums that are not finite: the wave does its tile again on the fp32
 //    matrix cores (plain), about five times slower.
-template <int NW, int FM, int BN, bool AK, bool BKC, bool FLUSH, int GC, int AB, int NV, int G = kGNone>
+template <int NW, int FM, int BN, bool AK, bool BKC, bool FLUSH, int GC, int AB, int NV, int G = kGNone, bool GU = false>
 struct SplitTile {
     static constexpr int NT = NW * kWave;
     static constexpr int BM = 16 * FM * NW, BK = 32;
@@ -55,6 +55,9 @@ struct SplitTile {
     static constexpr bool GATHER_K = G == kGNhwc || G == kGTransposed;  // convolutions: B gathered K-contiguously
     static constexpr bool GATHER_X = G == kGNhwcW;                      // ... or X-contiguously
     static_assert(G == kGNone || (GATHER_K && BKC) || (GATHER_X && !BKC), "the NHWC gathers");
+    // GU: every slice of K lies in one filter tap (GATHER_K: channels are a multiple of 32), or every aligned run of 4 of
+    // K in one output row (GATHER_X: out_w a multiple of 4).  A kernel of its own for each, and offsets made without a
+    // branch: a branch inside a step ends the region that interleave() orders.
     static constexpr int kNoRow = -(1 << 30);  // an image row that no tap reaches
 
     // slot of chunk c (8 k, 16 bytes) of LDS row r: the chunks of 4 rows fill the 64 banks, and the rotation spreads the
@@ -118,8 +121,10 @@ struct SplitTile {
             lpos[j] = slot(row, c);
             if constexpr (GATHER_K) {
                 const int oh = zn_udiv(x, cg.ow_mul, cg.ow_shift), ow = x - oh * cg.out_w;
-                gh[j] = x >= p.n ? kNoRow : G == kGNhwc ? oh * cg.stride_h - cg.pad_h : oh + cg.pad_h;
+                const int ih = G == kGNhwc ? oh * cg.stride_h - cg.pad_h : oh + cg.pad_h;
                 gw[j] = G == kGNhwc ? ow * cg.stride_w - cg.pad_w : ow + cg.pad_w;
+                gh[j] = x < p.n ? ih : kNoRow;
+                offb[j] = (uint32_t)((ih * cg.in_w + gw[j]) * cg.channels + (GU ? kq[j] : 0)) * 4u;
             }
             if constexpr (GATHER_X) {
                 const int khw = zn_udiv(x, cg.div1_mul, cg.div1_shift), ic = x - khw * cg.div1;
@@ -150,7 +155,7 @@ struct SplitTile {
                     for (int e = 0; e < 8; ++e)
                         g[e] = __builtin_bit_cast(
                             float, __builtin_amdgcn_raw_buffer_load_b32(
-                                       ra, offa[f], (uint32_t)(k0 + (e < 4 ? e : 12 + e)) * (uint32_t)lda * 4u, 0));
+                                       ra, offa[f], (uint32_t)(k0 * lda) * 4u + (uint32_t)((e < 4 ? e : 12 + e) * lda) * 4u, 0));
                 } else {
                     // k rows past the end: the last row (zeroed below)
 #pragma unroll
@@ -162,30 +167,36 @@ struct SplitTile {
                 }
             }
         };
-        // byte offset of channel ic under tap (kh, kw) of unit j's pixel, or out of range in the padding
-        auto gather_k = [&](int j, int kh, int kw, int ic) {
+        // byte offset of the value `at` places from unit j's pixel, under tap (kh, kw), or out of range in the padding
+        auto gather_k = [&](int j, int kh, int kw, uint32_t at) {
             const int ih = G == kGNhwc ? gh[j] + kh : gh[j] - kh, iw = G == kGNhwc ? gw[j] + kw : gw[j] - kw;
-            const bool ok = (unsigned)ih < (unsigned)cg.in_h && (unsigned)iw < (unsigned)cg.in_w;
-            return ok ? (uint32_t)((ih * cg.in_w + iw) * cg.channels + ic) * 4u : kOutOfRange;
+            const bool ok = ((unsigned)ih < (unsigned)cg.in_h) & ((unsigned)iw < (unsigned)cg.in_w);
+            const uint32_t off = offb[j] + at * 4u;
+            return ok ? off : kOutOfRange;
+        };
+        auto tap_k = [&](int k, int &kh, int &kw) {  // places from a pixel to the one under k's tap, at k's channel
+            const int khw = zn_udiv(k, cg.div1_mul, cg.div1_shift);
+            kh = zn_udiv(khw, cg.kw_mul, cg.kw_shift);
+            kw = khw - kh * cg.k_w;
+            const int px = kh * cg.in_w + kw;
+            return (uint32_t)((G == kGNhwc ? px : -px) * cg.channels + k - khw * cg.div1);
         };
         auto load_b = [&](int s, int j, float(&g)[8]) {
             if constexpr (GATHER_K) {
-                // 4 consecutive channels of one tap a load (channels are a multiple of 4); tap_uniform: the whole slice
-                // lies in one tap, decoded on the scalar unit
+                // 4 consecutive channels of one tap a load (channels are a multiple of 4); GU: the tap on the scalar unit
                 const int k0 = kbeg + s * BK;
                 uint32_t off[2];
-                if (cg.tap_uniform) {
-                    const int khw = zn_udiv(k0, cg.div1_mul, cg.div1_shift);
-                    const int kh = zn_udiv(khw, cg.kw_mul, cg.kw_shift);
-                    off[0] = gather_k(j, kh, khw - kh * cg.k_w, k0 - khw * cg.div1 + kq[j]);
+                int kh, kw;
+                if constexpr (GU) {
+                    const uint32_t at = tap_k(k0, kh, kw);
+                    off[0] = gather_k(j, kh, kw, at);
                     off[1] = off[0] + 64;
                 } else {
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         const int k = k0 + kq[j] + 16 * h;
-                        const int khw = zn_udiv(k, cg.div1_mul, cg.div1_shift);
-                        const int kh = zn_udiv(khw, cg.kw_mul, cg.kw_shift);
-                        off[h] = k < kend ? gather_k(j, kh, khw - kh * cg.k_w, k - khw * cg.div1) : kOutOfRange;
+                        const uint32_t at = tap_k(k, kh, kw), o = gather_k(j, kh, kw, at);
+                        off[h] = k < kend ? o : kOutOfRange;
                     }
                 }
 #pragma unroll
@@ -195,38 +206,44 @@ struct SplitTile {
                     for (int e = 0; e < 4; ++e) g[4 * h + e] = v[e];
                 }
             } else if constexpr (GATHER_X) {
-                // 64 channels-under-a-tap of one output pixel a load; the pixel is wave-uniform.  Rows of whole quads of
-                // pixels: one decode for each 4 consecutive pixels.
+                // 64 channels-under-a-tap of one output pixel a load; the pixel is wave-uniform.  GU: one decode for each 4
+                // consecutive pixels, which share their row.
                 const int plane = cg.channels * cg.in_h * cg.in_w;
                 uint32_t off[8];
-                auto pixel = [&](int k, int &base, int &oh, int &ow) {
-                    k = min(k, kend - 1);  // pixels past the end meet zeros of A
+                // pixel k (the last ones instead of those past the end, which meet zeros of A): its first row and column of
+                // the image, and the place of that value
+                auto pixel = [&](int k, int &oh, int &ow) {
+                    k = min(k, kend - (GU ? 4 : 1));
                     const int q = zn_udiv(k, cg.ow_mul, cg.ow_shift);
                     const int b = zn_udiv(q, cg.oh_mul, cg.oh_shift);
                     ow = (k - q * cg.out_w) * cg.stride_w;
                     oh = (q - b * cg.out_h) * cg.stride_h;
-                    base = b * plane + (oh * cg.in_w + ow) * cg.channels;
-                };
-                auto place = [&](int base, int oh, int ow) {
-                    const bool ok = (unsigned)(gh[j] + oh) < (unsigned)cg.in_h && (unsigned)(gw[j] + ow) < (unsigned)cg.in_w;
-                    return ok ? offb[j] + (uint32_t)base * 4u : kOutOfRange;
+                    return (uint32_t)(b * plane + (oh * cg.in_w + ow) * cg.channels) * 4u;
                 };
                 const int k0 = kbeg + s * BK + kq[j];
-                if (cg.out_w % 4 == 0) {
+                if constexpr (GU) {
+                    const uint32_t next = (uint32_t)(cg.stride_w * cg.channels) * 4u;
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
-                        int base, oh, ow;
-                        pixel(k0 + 16 * h, base, oh, ow);
+                        int oh, ow;
+                        const uint32_t at = pixel(k0 + 16 * h, oh, ow);
+                        const bool row = (unsigned)(gh[j] + oh) < (unsigned)cg.in_h;
+                        const uint32_t o = row ? offb[j] + at : kOutOfRange;
+                        const int iw = gw[j] + ow;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            off[4 * h + e] = place(base + e * cg.stride_w * cg.channels, oh, ow + e * cg.stride_w);
+                        for (int e = 0; e < 4; ++e) {
+                            const uint32_t oe = o + e * next;
+                            off[4 * h + e] = (unsigned)(iw + e * cg.stride_w) < (unsigned)cg.in_w ? oe : kOutOfRange;
+                        }
                     }
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        int base, oh, ow;
-                        pixel(k0 + (e < 4 ? e : 12 + e), base, oh, ow);
-                        off[e] = place(base, oh, ow);
+                        int oh, ow;
+                        const uint32_t at = pixel(k0 + (e < 4 ? e : 12 + e), oh, ow);
+                        const bool ok = ((unsigned)(gh[j] + oh) < (unsigned)cg.in_h) & ((unsigned)(gw[j] + ow) < (unsigned)cg.in_w);
+                        const uint32_t o = offb[j] + at;
+                        off[e] = ok ? o : kOutOfRange;
                     }
                 }
 #pragma unroll

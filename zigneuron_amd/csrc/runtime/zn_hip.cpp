@@ -190,7 +190,7 @@ struct zn_ctx {
     hipFunction_t dense_bwd_k[2] = {};         // the same on 32x32 tiles with K split over 4 waves [16-byte]
     hipFunction_t convf[kNumTiles][2] = {};    // convolution forward on NHWC [tile][16-byte W rows]
     hipFunction_t convwn[kNumTiles][2] = {};   // weight gradient on NHWC [tile][16-byte grad_output rows]
-    hipFunction_t conv_split[3][2] = {};       // [forward, input, weight gradient][cr, ch]: the bf16 matrix cores
+    hipFunction_t conv_split[3][2][2] = {};    // [forward, input, weight gradient][cr, ch][_u]: the bf16 matrix cores
     hipFunction_t gemmp[3][kNumTiles] = {};    // persistent plain GEMM, 16-byte staging [layout][tile] (not s)
     hipFunction_t gemmk[3][2][2] = {};         // intra-workgroup split-K, 32x32 tiles [layout][4 or 8 waves][16-byte]
     int gemmp_occ[3][kNumTiles] = {};          // its resident workgroups per CU
@@ -966,8 +966,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     args.bias_rows = bias_rows ? 1 : 0;
     if (conv) args.conv = *conv;
     // NHWC forward: each BK slice of K lies in one filter tap when the channels are whole slices
-    if (conv && (mode == kGatherNhwc || (conv_split && mode == kGatherTransposed)))
-        args.conv.tap_uniform = conv->channels % ts.bk == 0 ? 1 : 0;
+    if (conv && mode == kGatherNhwc) args.conv.tap_uniform = conv->channels % ts.bk == 0 ? 1 : 0;
     // 16-byte staging: aligned rows and contiguous extents that are whole float4s
     const bool vec = conv ? (aligned16(a) && lda % 4 == 0 && stride_a % 4 == 0 && a_row % 4 == 0)
                           : (aligned16(a) && aligned16(b) && lda % 4 == 0 && ldb % 4 == 0 && stride_a % 4 == 0 &&
@@ -1042,7 +1041,9 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // 4-pixel (16-byte) gather: unit column stride, and whole chunks of 4 pixels per output row
     const int gather4 = conv && conv->stride_w == 1 && conv->out_w % 4 == 0 ? 1 : 0;
     const int staging = bf16x3 ? 0 : unaligned ? 2 : vec ? 1 : 0;  // 4-byte (split: any), 16-byte, 16-byte unaligned
-    hipFunction_t f = conv_split ? ctx->conv_split[mode == kGatherNhwc ? 0 : mode == kGatherTransposed ? 1 : 2][tile - kTileCR]
+    // gathers that make one decode of each K slice (the filter tap) or of each 4 of K (the output row)
+    const int conv_uniform = conv && (mode == kGatherWeightNhwc ? conv->out_w % 4 == 0 : conv->channels % ts.bk == 0) ? 1 : 0;
+    hipFunction_t f = conv_split ? ctx->conv_split[mode == kGatherNhwc ? 0 : mode == kGatherTransposed ? 1 : 2][tile - kTileCR][conv_uniform]
                       : !conv                     ? ctx->gemm[layout][tile][staging]
                       : mode == kGatherTransposed ? ctx->convt[tile][vec ? 1 : 0]
                       : mode == kGatherWeightGrad ? ctx->convw[tile][vec ? 1 : 0]
@@ -1831,13 +1832,14 @@ int zn_hip_create(int device, const char *code_object_dir, zn_ctx **out) {
     if (hipModuleGetFunction(&ctx->convwn[kTileR][1], ctx->conv_module, "zn_convwn_tn_r_v") != hipSuccess)
         return bail(ZN_ERR_SYMBOL);
     for (int g = 0; g < 3; ++g)
-        for (int t = 0; t < 2; ++t) {
-            static const char *kFamily[3] = {"zn_convfs_nt", "zn_convts_nt", "zn_convwns_tn"};
-            char name[64];
-            std::snprintf(name, sizeof(name), "%s_%s", kFamily[g], kTiles[kTileCR + t].suffix);
-            if (hipModuleGetFunction(&ctx->conv_split[g][t], ctx->conv_module, name) != hipSuccess)
-                return bail(ZN_ERR_SYMBOL);
-        }
+        for (int t = 0; t < 2; ++t)
+            for (int u = 0; u < 2; ++u) {
+                static const char *kFamily[3] = {"zn_convfs_nt", "zn_convts_nt", "zn_convwns_tn"};
+                char name[64];
+                std::snprintf(name, sizeof(name), "%s_%s%s", kFamily[g], kTiles[kTileCR + t].suffix, u ? "_u" : "");
+                if (hipModuleGetFunction(&ctx->conv_split[g][t][u], ctx->conv_module, name) != hipSuccess)
+                    return bail(ZN_ERR_SYMBOL);
+            }
     for (int l = 0; l < 3; ++l)
         for (int w = 0; w < 2; ++w)
             for (int v = 0; v < 2; ++v) {
