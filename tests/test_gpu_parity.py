@@ -605,3 +605,32 @@ def test_every_tile_strided_batched(ctx, tile):
         assert_close(c[i], ref_gemm("nt", a[i], b[i], m, n, k), "nt", a[i], b[i], m, n, k, what=f"{tile} {i}")
     for buf in (da, db, dc):
         buf.close()
+
+
+@pytest.mark.parametrize("splits", [16, 17, 64, 65, 66, 129, 250])
+@pytest.mark.parametrize("m,n,ldc,batch", [(3, 5, 7, 1), (64, 65, 65, 1), (1, 64, 64, 3), (17, 40, 44, 2)])
+def test_reduce_of_many_slices(ctx, splits, m, n, ldc, batch):
+    """Few values in many K slices are added by a kernel of their own, in slice order like the other: the same sums as
+    with a bias of zeros, which keeps the other (and, added last, changes no value)."""
+    rng = np.random.default_rng(splits * 1000 + m)
+    k = 32 * splits + 5
+    a, b, c0 = uniform(rng, (batch, m, k)), uniform(rng, (batch, k, n)), uniform(rng, (batch, m, ldc))
+    da, db, zero = ctx.to_device(a), ctx.to_device(b), ctx.to_device(np.zeros(n, np.float32))
+    announce(f"reduce of {splits} slices, {batch} x {m}x{n}, ldc {ldc}")
+    try:
+        ctx.set_gemm_splits(splits)
+        for accumulate in (False, True):
+            outs = []
+            for bias in (None, zero):
+                dc = ctx.to_device(c0)
+                ctx.sgemm_strided_batched("nn", m, n, k, da, k, m * k, db, n, k * n, dc, ldc, m * ldc, batch, accumulate, bias)
+                outs.append(dc.download().reshape(batch, m, ldc))
+                dc.close()
+            np.testing.assert_array_equal(outs[0], outs[1])
+            np.testing.assert_array_equal(outs[0][:, :, n:], c0[:, :, n:])
+            ref = a.astype(np.float64) @ b.astype(np.float64) + (c0[:, :, :n] if accumulate else 0)
+            assert np.abs(outs[0][:, :, :n] - ref).max() <= 1e-5 * np.sqrt(k) * np.abs(a).max() * np.abs(b).max() * 4
+    finally:
+        ctx.set_gemm_splits(0)
+    for buf in (da, db, zero):
+        buf.close()

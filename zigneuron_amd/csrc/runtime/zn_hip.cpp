@@ -75,13 +75,13 @@ constexpr TileShape kTiles[kNumTiles] = {{256, 128, 16, 512, "x", true, true, tr
                                          {64, 128, 32, 256, "ch", false, false, false}};
 constexpr const char *kLayoutName[3] = {"nn", "nt", "tn"};
 
-enum EltKernel { kFill, kCopy, kAddBias, kActFwd, kActBwd, kAccBias, kIm2col, kSoftmax, kCol2im, kRowSum, kDenseGrad, kRegroup, kPack, kToNhwc, kHold, kCol2imPx, kNumElt };
+enum EltKernel { kFill, kCopy, kAddBias, kActFwd, kActBwd, kAccBias, kIm2col, kSoftmax, kCol2im, kRowSum, kDenseGrad, kRegroup, kPack, kToNhwc, kHold, kCol2imPx, kReduceSlices, kNumElt };
 constexpr const char *kEltName[kNumElt] = {"zn_fill_f32",        "zn_copy_f32", "zn_add_bias",
                                            "zn_activation_forward", "zn_activation_backward",
                                            "zn_accumulate_bias", "zn_im2col",   "zn_softmax_rows",
                                            "zn_col2im",          "zn_row_sum",  "zn_dense_grad_prologue",
                                            "zn_weight_regroup", "zn_pack_rows", "zn_nchw_to_nhwc",
-                                           "zn_hold_stream",     "zn_col2im_px"};
+                                           "zn_hold_stream",     "zn_col2im_px", "zn_reduce_slices"};
 
 constexpr const char *kGemmObject = "zn_gemm_gfx950.hsaco";
 constexpr const char *kConvObject = "zn_conv_gfx950.hsaco";
@@ -513,6 +513,20 @@ int64_t round_splits(int64_t tiles, int64_t k, int64_t cus) {
 
 // The device's compute units, or MI355X's 256 when the query gave none.
 int64_t cus_now(const zn_ctx *ctx) { return ctx->info.compute_units > 0 ? ctx->info.compute_units : 256; }
+
+// C from r.splits slices of partial sums, added in slice order.  More than 16
+// slices of at most 512 values a CU take a thread a value with 64 slices'
+// loads in flight (MI355X: 256 slices of 1024 values 25 -> 8 us, 51 of 128 x
+// 576 6.4 -> 4.7; with 16 slices the same, 32 of 512 x 512 7.2 -> 7.4, and
+// where the values fill the chip by themselves it is slower: 8 of 1024 x 1024
+// 8.9 -> 19 us).
+int launch_reduce(zn_ctx *ctx, ZnReduceArgs &r) {
+    const int64_t mn = (int64_t)r.m * r.n, cus = cus_now(ctx);
+    if (r.splits > 16 && !r.bias && r.act == ZN_ACT_LINEAR && mn * r.batch <= 512 * cus)
+        return launch(ctx, ctx->elt[kReduceSlices], (unsigned)cdiv(mn, 64), (unsigned)r.batch, 64, &r);
+    const int64_t blocks = cdiv(mn * r.batch / (r.vec ? 4 : 1), 256);
+    return launch(ctx, ctx->splitk_reduce, (unsigned)std::min<int64_t>(blocks, 8 * cus), 1, 256, &r);
+}
 
 // Tile choice, from measurements on MI355X (256 CUs, per-launch times from
 // graph replays): the largest tiles win once they give every CU two or more
@@ -1234,12 +1248,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
             r.act = act;
             r.bias_rows = bias_rows ? 1 : 0;
             r.vec = (n % 4 == 0 && ldc % 4 == 0 && stride_c % 4 == 0 && aligned16(part.c)) ? 1 : 0;
-            const int64_t items = m * n * nb / (r.vec ? 4 : 1);
-            int64_t blocks = cdiv(items, 256);
-            const int64_t cap = cus_now(ctx) * 8;
-            if (blocks > cap) blocks = cap;
-            rc = launch(ctx, ctx->splitk_reduce, (unsigned)blocks, 1, 256, &r);
-            if (rc) return rc;
+            if ((rc = launch_reduce(ctx, r))) return rc;
         }
     }
     return ZN_OK;
@@ -2661,7 +2670,7 @@ static int dense_backward_impl(zn_ctx *ctx, int act, const float *input, const f
                 return zn_hip_activation_backward(ctx, prev_act, prev_y, grad_input, prev_gaa, batch * in_size);
             return ZN_OK;
         }
-        if ((rc = launch(ctx, ctx->splitk_reduce, (unsigned)blocks, 1, 256, &r))) return rc;
+        if ((rc = launch_reduce(ctx, r))) return rc;
     }
     if (in_size == 0) return ZN_OK;
     if (grad_input && batch > 0 &&
@@ -2995,10 +3004,7 @@ static int conv2d_backward_device(zn_ctx *ctx, const float *input, const float *
             r.accumulate = b0 > 0;
             r.act = ZN_ACT_LINEAR;
             r.vec = (taps % 4 == 0 && aligned16(grad_weights) && aligned16(part.ptr)) ? 1 : 0;
-            int64_t blocks = cdiv(oc * taps / (r.vec ? 4 : 1), 256);
-            const int64_t cap = cus_now(ctx) * 8;
-            if (blocks > cap) blocks = cap;
-            if ((rc = launch(ctx, ctx->splitk_reduce, (unsigned)blocks, 1, 256, &r))) return rc;
+            if ((rc = launch_reduce(ctx, r))) return rc;
             // grad_col_b = go_b^T . W: TN, M = HW, N = taps, K = OC, per image
             if ((rc = gemm_launch(ctx, ZN_LAYOUT_TN, hw, taps, oc, go, hw, oc * hw, weights, taps, 0, col.ptr, taps,
                                   hw * taps, nb, 0, nullptr, ZN_ACT_LINEAR)))
@@ -3063,7 +3069,7 @@ static int conv2d_backward_device(zn_ctx *ctx, const float *input, const float *
     r.batch = 1;
     r.splits = (int32_t)batch;
     r.act = ZN_ACT_LINEAR;
-    return launch(ctx, ctx->splitk_reduce, (unsigned)std::min<int64_t>(cdiv(oc, 256), cap), 1, 256, &r);
+    return launch_reduce(ctx, r);
 }
 
 int zn_hip_col2im(zn_ctx *ctx, const float *col, float *output, int64_t batch, int64_t channels, int64_t in_h,
