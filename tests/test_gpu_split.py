@@ -225,3 +225,36 @@ def test_split_convolutions(ctx, case, poison):
         check(gx.download().reshape(B, C, H, W).transpose(0, 2, 3, 1), ref[inner], den[inner], taps // C * OC, "input gradient")
     for b in (dx, dw, db, dg, y, gx, gw, gb):
         b.close()
+
+
+def test_split_convolution_non_finite_far_into_a_long_col(ctx):
+    """One image of 512 x 512 x 256 under 3x3: its col matrix has more than 2^29 values, and value (pixel 455 * 512 + 56,
+    tap (2, 2) of channel 0) is number 2^29, byte 2^31.  An Inf there reaches exactly the outputs, input gradients and
+    weight gradients that it reaches in the reference's im2col (src/backend.zig:3881-4065).  Everything else is 1, so
+    every other value is a count, exact in fp32 in any order."""
+    C, H, W = 256, 512, 512
+    assert (455 * W + 56) * 9 * C + 8 * C == 2 ** 29
+    dx, dg = ctx.alloc(C * H * W).fill(1.0), ctx.alloc(H * W * C).fill(1.0)
+    dw, db = ctx.alloc(C * 9 * C).fill(1.0), ctx.alloc(C).fill(0.0)
+    y, gx, gw, gb = (ctx.alloc(n).fill(0.5) for n in (C * H * W, C * H * W, C * 9 * C, C))
+    inf = ctx.to_device(np.full(1, np.inf, np.float32))
+    ctx.copy(dx.offset(456 * W + 57), inf.ptr, 1)        # channel 0 (NCHW)
+    ctx.copy(dg.offset((454 * W + 55) * C), inf.ptr, 1)  # output channel 0 ([pixel][channel])
+    geom = (1, C, C, 3, 3, H, W, H, W, 1, 1, 1, 1)
+    announce("split convolution, Inf at byte 2^31 of col")
+    ctx.conv2d_forward_im2col(dx, dw, db, y, *geom)
+    ctx.conv2d_backward_im2col(dx, dw, dg, gx, gw, gb, *geom)
+    rows = np.r_[2.0, np.full(H - 2, 3.0), 2.0]  # taps that lie in the image
+    want = np.outer(rows, rows).astype(np.float32) * C
+    fwd, back = want.copy(), want.copy()
+    fwd[455:458, 56:59] = np.inf
+    back[453:456, 54:57] = np.inf
+    for got, ref, what in ((y, fwd, "forward"), (gx, back, "input gradient")):
+        got = got.download().reshape(C, H, W)
+        assert all(np.array_equal(got[c], ref) for c in range(C)), what
+    span = np.r_[H - 1.0, H, H - 1.0]
+    wgrad = np.broadcast_to(np.outer(span, span).reshape(1, 9, 1), (C, 9, C)).astype(np.float32).copy()
+    wgrad[0], wgrad[:, :, 0] = np.inf, np.inf
+    np.testing.assert_array_equal(gw.download().reshape(C, 9, C), wgrad)
+    for b in (dx, dg, dw, db, y, gx, gw, gb, inf):
+        b.close()

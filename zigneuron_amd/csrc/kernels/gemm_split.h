@@ -415,8 +415,13 @@ struct SplitTile {
 #pragma unroll
             for (int f = 0; f < FN; ++f) {
                 const int x = nw + 16 * f + li;
-                uint32_t off = x < p.n && kk < kend ? (uint32_t)(BKC ? x * ldb + kk : kk * ldb + x) * 4u : kOutOfRange;
-                if constexpr (G != kGNone) {
+                const bool in = x < p.n && kk < kend;
+                uint32_t off;
+                if constexpr (G == kGNone) {
+                    off = in ? (uint32_t)(BKC ? x * ldb + kk : kk * ldb + x) * 4u : kOutOfRange;
+                } else {
+                    // only the gathered operand's own extent is bounded: the col matrix it stands for has pixels x taps
+                    // values, whose offsets may pass 2^31 and meet kOutOfRange
                     const ZnConvGeom &cg = p.conv;
                     const int px = GATHER_X ? kk : x, tap = GATHER_X ? x : kk;
                     const int khw = zn_udiv(tap, cg.div1_mul, cg.div1_shift), ic = tap - khw * cg.div1;
@@ -425,7 +430,7 @@ struct SplitTile {
                     const int img = GATHER_X ? zn_udiv(q, cg.oh_mul, cg.oh_shift) : 0, oh = q - img * cg.out_h;
                     const int ih = G == kGTransposed ? q + cg.pad_h - kh : (GATHER_X ? oh : q) * cg.stride_h - cg.pad_h + kh;
                     const int iw = G == kGTransposed ? ow + cg.pad_w - kw : ow * cg.stride_w - cg.pad_w + kw;
-                    const bool ok = off != kOutOfRange && (unsigned)ih < (unsigned)cg.in_h && (unsigned)iw < (unsigned)cg.in_w;
+                    const bool ok = in && (unsigned)ih < (unsigned)cg.in_h && (unsigned)iw < (unsigned)cg.in_w;
                     off = ok ? (uint32_t)(((img * cg.in_h + ih) * cg.in_w + iw) * cg.channels + ic) * 4u : kOutOfRange;
                 }
                 b[f] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, off, 0, 0));
