@@ -167,6 +167,31 @@ def test_split_padded_rows_accumulate_batches(ctx, layout):
         buf.close()
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_forced_tile_takes_the_named_kernel(ctx, layout):
+    """zn_hip_set_gemm_tile at a size that the policy gives to the split kernels (4096 x 1024 x 512): the fp32 tiles agree
+    bit for bit with each other and not with the policy's result, the split tile does."""
+    m, n, k = 4096, 1024, 512
+    rng = np.random.default_rng(21)
+    a_shape, b_shape = stored_shapes(layout, m, n, k)
+    a, b = uniform(rng, a_shape), uniform(rng, b_shape)
+    out = {}
+    try:
+        ctx.set_gemm_splits(1)
+        for tile in ("auto", "128x128", "64x64", "256x256", "128x128s", "128x64s"):
+            announce(f"forced {tile} {layout}")
+            ctx.set_gemm_tile(tile)
+            out[tile] = run_gemm(ctx, layout, a, b, m, n, k).view(np.uint32)
+    finally:
+        ctx.set_gemm_tile("auto")
+        ctx.set_gemm_splits(0)
+    np.testing.assert_array_equal(out["128x128"], out["64x64"])
+    np.testing.assert_array_equal(out["128x128"], out["256x256"])
+    np.testing.assert_array_equal(out["128x128s"], out["auto"])
+    np.testing.assert_array_equal(out["128x64s"], out["auto"])
+    assert not np.array_equal(out["128x128"], out["auto"])
+
+
 CONVS = [(4, 64, 56, 56, 128, 3, 1, 1),   # channels a multiple of 32: one tap per K slice
          (16, 36, 33, 35, 100, 3, 1, 1),  # taps change inside a slice; rows of 35 pixels
          (16, 32, 61, 59, 48, 5, 2, 2),   # stride 2, 64-row tiles

@@ -179,12 +179,13 @@ def test_unaligned_strided_batches(ctx, layout):
 @pytest.mark.parametrize("layout,mode", [(lay, mode) for lay in ("nn", "nt", "tn") for mode in ("plain", "accumulate")]
                          + [("nn", "bias_relu")])  # the fused bias epilogue is Backend.matMulBias*, NN only
 def test_row_tail_folded_into_unaligned_launch(ctx, layout, mode):
-    """C4's 4097 x 1023 x 777: the automatic choice runs rows 0..4095 on the
-    unaligned 128x128 tiles and the last row as dot products inside the same
+    """4097 x 1023 x 255, just below the 2^30 multiply-adds (and the K of 256)
+    from which such a problem runs on split operands: the automatic choice runs
+    rows 0..4095 on the unaligned 128x128 tiles and the last row as dot products inside the same
     launch.  The first 4096 rows are bit-identical to one launch of the same
     kernel over all rows (forcing the tile turns the row split off); the last
     row and sampled rows match the oracle."""
-    m, n, k = 4097, 1023, 777
+    m, n, k = 4097, 1023, 255
     rng = np.random.default_rng(10 * "nn nt tn".split().index(layout) + "plain accumulate bias_relu".split().index(mode))
     a_shape, b_shape = stored_shapes(layout, m, n, k)
     a, b = uniform(rng, a_shape), uniform(rng, b_shape)

@@ -117,9 +117,10 @@ def test_noalloc_unaligned_rows_are_not_packed(ctx):
 
 
 def test_noalloc_split_beyond_scratch(ctx):
-    """4097^2 x 4096 NN: the policy splits K three ways (201 MiB of partial
-    sums, more than the scratch), so the no-allocation GEMM runs unsplit:
-    within the tolerance of the oracle.  A forced split that needs more than
+    """4097^2 x 4096 NN on 256x128 fp32 tiles: the policy splits K three ways
+    (201 MiB of partial sums, more than the scratch), so the no-allocation GEMM
+    runs unsplit (another order of the same sums: other bits), within the
+    tolerance of the oracle.  A forced split that needs more than
     the scratch is refused; one that fits matches zn_hip_sgemm bit for bit."""
     from zigneuron_amd import InvalidArgumentError
     rng = np.random.default_rng(79)
@@ -127,7 +128,12 @@ def test_noalloc_split_beyond_scratch(ctx):
     k = 4096
     a, b = uniform(rng, (m, k)), uniform(rng, (k, n))
     announce("noalloc NN 4097x4097x4096 (policy split beyond the scratch)")
-    _, got = run_both(ctx, "nn", m, n, k, a, b)
+    ctx.set_gemm_tile("256x128")
+    try:
+        split, got = run_both(ctx, "nn", m, n, k, a, b)
+    finally:
+        ctx.set_gemm_tile("auto")
+    assert not np.array_equal(got, split)
     assert_close(got, ref_gemm("nn", a, b, m, n, k), "nn", a, b, m, n, k, what="noalloc unsplit")
     m2, n2, k2 = 1024, 1024, 4096
     a2, b2 = uniform(rng, (m2, k2)), uniform(rng, (k2, n2))

@@ -48,10 +48,8 @@ namespace {
 
 // Macro tiles of the GEMM code object (kernels/gemm_f32.hip).
 // The last six run on the bf16 matrix cores (three-way split operands,
-// kernels/gemm_split.h) and are chosen by size alone (split_pays); cr and ch
-// are the convolutions'.
+// kernels/gemm_split.h); cr and ch are the convolutions'.
 enum Tile { kTileX = 0, kTileL, kTileN, kTileM, kTileS, kTileR, kTileH, kTileW, kTileSW, kTileSX, kTileSR, kTileSN, kTileCR, kTileCH, kNumTiles };
-constexpr int kNumUserTiles = kTileSW;  // zn_hip_set_gemm_tile
 struct TileShape {
     int bm, bn, bk, threads;
     const char *suffix;
@@ -690,8 +688,7 @@ int64_t split_main_rows(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int6
 }
 
 // Whether a problem runs on the split kernels: by its size alone, so that
-// every forced tile, every row chunk and every staging of the same problem
-// gives the same sums.  K below 256 is left to the fp32 kernels (its time is
+// every staging of the same problem gives the same sums.  K below 256 is left to the fp32 kernels (its time is
 // mostly stores), and so is less than 2^30 multiply-adds, where one round of
 // 64x64 fp32 tiles is as fast (MI355X, 1000^3: 24.1 us split, 24.3 us fp32).
 // Above, the estimate is set against what the fp32 kernels reach: about 125
@@ -817,8 +814,15 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
 
     // The NHWC forward gather runs best on 64x64 tiles (C5 forward, rocprofv3 trace: 156 us against 172 us for
     // 128x128 and 314 us for 256x128).
-    // A forced tile without convolution kernels leaves convolutions to the policy.
-    const bool forced = ctx->forced_tile >= 0 && (!conv || kTiles[ctx->forced_tile].conv);
+    // A forced tile without convolution kernels (of this gather) leaves convolutions to the policy, one with no others
+    // (cr, ch) plain GEMMs; the split kernels and the wave splits take no sums of nothing, and a forced wave split is
+    // an fp32 form.
+    const bool split_gather = conv && (mode == kGatherNhwc || mode == kGatherTransposed || mode == kGatherWeightNhwc);
+    const bool forced = ctx->forced_tile < 0          ? false
+                        : ctx->forced_tile >= kTileCR ? split_gather && k > 0
+                        : conv                        ? kTiles[ctx->forced_tile].conv
+                        : ctx->forced_tile >= kTileSW ? k > 0 && ctx->forced_wave_split <= 0
+                                                      : true;
     // 16-byte staging of both operands as they lie (the tiles without a
     // 4-byte kernel need it; packed copies are not made for them)
     const bool native_vec = !conv && aligned16(a) && aligned16(b) && lda % 4 == 0 && ldb % 4 == 0 && stride_a % 4 == 0 &&
@@ -834,33 +838,35 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
                 : conv && mode == kGatherNhwc ? kTileM
                 : wn_wide                     ? kTileR
                                               : choose_tile(ctx, m, n, k, batch, conv != nullptr, native_vec);
-    if (!kTiles[tile].plain && !native_vec) tile = kTileX;  // forced onto a tile it cannot stage: 256x128
-    // The split kernels, by size (forced wave splits and persistent kernels are fp32 forms)
-    const bool bf16x3 = !conv && k > 0 && ctx->forced_wave_split <= 0 && ctx->forced_persistent < 0 &&
-                        (arith == 1 || (arith < 0 && split_pays(ctx, m, n, k, batch)));
-    int policy_splits = 0;
+    if (!conv && !kTiles[tile].plain && !native_vec) tile = kTileX;  // forced onto a tile it cannot stage: 256x128
+    // The split kernels: a forced tile, or by size (forced wave splits and persistent kernels are fp32 forms)
+    const bool by_size = !forced && k > 0 && ctx->forced_wave_split <= 0 && ctx->forced_persistent < 0;
+    const bool bf16x3 = !conv && (forced ? tile >= kTileSW
+                                         : by_size && (arith == 1 || (arith < 0 && split_pays(ctx, m, n, k, batch))));
+    int policy_splits = 1;
     const bool conv_policy = conv && !forced && ctx->forced_splits == 0 && ctx->forced_persistent < 0 && k > 0;
-    bool conv_split = false;
-    if (conv_policy && (mode == kGatherNhwc || mode == kGatherTransposed)) {
+    bool conv_split = conv && forced && tile >= kTileCR;
+    // few tiles over every output pixel: K slices for one round of workgroups
+    auto weight_slices = [&](Tile t) {
+        const int64_t tiles = cdiv(m, kTiles[t].bm) * cdiv(n, kTiles[t].bn);
+        return (int)std::max<int64_t>(1, std::min<int64_t>({64, cus_now(ctx) / tiles, k / 768}));
+    };
+    if (conv_split) {
+        if (mode == kGatherWeightNhwc) policy_splits = weight_slices(tile);
+    } else if (conv_policy && (mode == kGatherNhwc || mode == kGatherTransposed)) {
         const Tile t = conv_split_tile(ctx, m, n, k, batch, 1);
-        if ((conv_split = t != kNumTiles)) {
-            tile = t;
-            policy_splits = 1;
-        }
+        if ((conv_split = t != kNumTiles)) tile = t;
     } else if (conv_policy && mode == kGatherWeightNhwc && k >= 64 * 128) {
-        // few tiles over every output pixel: K slices for one round of workgroups
-        const int64_t tiles = cdiv(m, 128) * cdiv(n, 128);
-        const int64_t s = std::max<int64_t>(1, std::min<int64_t>({64, cus_now(ctx) / tiles, k / 768}));
-        if ((conv_split = conv_split_tile(ctx, m, n, k, 1, s) != kNumTiles)) {
+        if ((conv_split = conv_split_tile(ctx, m, n, k, 1, weight_slices(kTileCR)) != kNumTiles)) {
             tile = m > 64 ? kTileCR : kTileCH;
-            policy_splits = (int)std::max<int64_t>(1, std::min<int64_t>({64, cus_now(ctx) / (cdiv(m, kTiles[tile].bm) * cdiv(n, 128)), k / 768}));
+            policy_splits = weight_slices(tile);
         }
     }
-    if (bf16x3) {
+    if (bf16x3 && !forced) {
         // part of a larger problem: the sums of the whole, which K slices would change
         SplitChoice ch = estimate_split(ctx, m, n, k, batch, arith == 1 ? 0 : (int64_t)kScratchBytes);
         const int64_t m_main = split_main_rows(ctx, m, n, k, batch, ch);
-        if (split_rows && m_main < m && ctx->forced_tile < 0 && ctx->forced_splits == 0) {
+        if (split_rows && m_main < m && ctx->forced_splits == 0) {
             const float *a_tail = layout == ZN_LAYOUT_TN ? a + m_main : a + m_main * lda;
             const int rc = gemm_launch_ex(ctx, layout, m_main, n, k, a, lda, 0, b, ldb, 0, c, ldc, 0, 1, accumulate, bias, act,
                                           bias_rows, nullptr, mode, false, padded, nullptr, 1);
@@ -1794,7 +1800,7 @@ int zn_hip_create(int device, const char *code_object_dir, zn_ctx **out) {
     }
     for (int l = 0; l < 3; ++l)
         for (int t = 0; t < kNumTiles; ++t)
-            for (int v = kTiles[t].plain ? 0 : 1; t < kTileCR && v < (t == kTileR ? 3 : t >= kNumUserTiles ? 1 : 2); ++v) {
+            for (int v = kTiles[t].plain ? 0 : 1; t < kTileCR && v < (t == kTileR ? 3 : t >= kTileSW ? 1 : 2); ++v) {
                 char name[64];
                 std::snprintf(name, sizeof(name), "zn_sgemm_%s_%s%s", kLayoutName[l], kTiles[t].suffix,
                               v == 2 ? "_u" : v ? "_v" : "");
@@ -2210,7 +2216,7 @@ int zn_hip_event_destroy(zn_event *ev) {
 
 // ------------------------------------------------------------------ GEMM
 int zn_hip_set_gemm_tile(zn_ctx *ctx, int tile) {
-    if (!ctx || tile < ZN_TILE_AUTO || tile >= kNumUserTiles) return ZN_ERR_INVALID_ARG;
+    if (!ctx || tile < ZN_TILE_AUTO || tile >= kNumTiles) return ZN_ERR_INVALID_ARG;
     ctx->forced_tile = tile;
     return ZN_OK;
 }
