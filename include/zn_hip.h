@@ -182,12 +182,13 @@ int zn_hip_event_destroy(zn_event *ev);
 #define ZN_TILE_64x64_K16 6   /* 64x64, BK 16, six workgroups per CU; not for convolutions */
 #define ZN_TILE_256x256 7     /* 256x256, BK 16, one workgroup per CU; 16-byte rows only (otherwise 256x128); not for
                                  convolutions */
-#define ZN_TILE_256x256_S 8   /* split operands, any alignment (8 to 11); K > 0; not for convolutions */
+#define ZN_TILE_256x256_S 8   /* split operands, any alignment (8 to 12); K > 0; not for convolutions */
 #define ZN_TILE_256x128_S 9
 #define ZN_TILE_128x128_S 10
 #define ZN_TILE_128x64_S 11
-#define ZN_TILE_CONV_128x128_S 12 /* convolutions gathered from NHWC images or grad_output rows only; other GEMMs and */
-#define ZN_TILE_CONV_64x128_S 13  /* convolutions are left to the policy */
+#define ZN_TILE_128x128_SC 12 /* the sums of 256x256_S, bit for bit */
+#define ZN_TILE_CONV_128x128_S 13 /* convolutions gathered from NHWC images or grad_output rows only; other GEMMs and */
+#define ZN_TILE_CONV_64x128_S 14  /* convolutions are left to the policy */
 int zn_hip_set_gemm_tile(zn_ctx *ctx, int tile);
 /* Split-K override: 0 (the default) lets the policy choose, 1..256 asks for
  * that many K slices (at most ceil(K / BK)) for every following GEMM on this

@@ -192,6 +192,43 @@ def test_forced_tile_takes_the_named_kernel(ctx, layout):
     assert not np.array_equal(out["128x128"], out["auto"])
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("tiles", [("256x256s", "128x128sc"), ("256x128s", "128x128s", "128x64s")], ids=["chain", "flush"])
+def test_split_tiles_agree_bit_for_bit(ctx, layout, tiles):
+    """The split tiles of one kind of sum, at an extent past each one's tiles and with a K tail."""
+    m, n, k = 391, 277, 165
+    rng = np.random.default_rng(22)
+    a, b = uniform(rng, (m, k)), uniform(rng, (k, n))
+    ast, bst = np.ascontiguousarray(as_mk(a, layout)), np.ascontiguousarray(as_kn(b, layout))
+    out = []
+    try:
+        for tile in tiles:
+            announce(f"tiles agree {layout} {tile}")
+            ctx.set_gemm_tile(tile)
+            out.append(run_gemm(ctx, layout, ast, bst, m, n, k).view(np.uint32))
+    finally:
+        ctx.set_gemm_tile("auto")
+    for other in out[1:]:
+        np.testing.assert_array_equal(out[0], other)
+
+
+@pytest.mark.parametrize("m,n,k", [(4096, 4096, 2048),   # 256x256 tiles; the chunks have 1024 rows
+                                   (4097, 1023, 1100)])  # 128x128 tiles and a one-row tail; three chunks
+def test_chunked_host_call_has_the_bits_of_the_device_call(ctx, m, n, k):
+    """Backend.matMul cuts a large A into row chunks, which take the tiles of their own size and the whole call's kind of
+    sum."""
+    from zigneuron_amd import Backend
+    rng = np.random.default_rng(m + k)
+    a, b = uniform(rng, (m, k)), uniform(rng, (k, n))
+    announce(f"chunked host call {m}x{n}x{k}")
+    backend = Backend.init(0)
+    for layout, name, rhs in (("nn", "matMul", b), ("nt", "matMulTransposeB", np.ascontiguousarray(b.T))):
+        host = np.empty((m, n), np.float32)
+        getattr(backend, name)(a, rhs, host, m, n, k)
+        np.testing.assert_array_equal(host, run_gemm(ctx, layout, a, rhs, m, n, k), err_msg=name)
+    backend.deinit()
+
+
 CONVS = [(4, 64, 56, 56, 128, 3, 1, 1),   # channels a multiple of 32: one tap per K slice
          (16, 36, 33, 35, 100, 3, 1, 1),  # taps change inside a slice; rows of 35 pixels
          (16, 32, 61, 59, 48, 5, 2, 2),   # stride 2, 64-row tiles

@@ -27,7 +27,8 @@ ZN_ERR_OVERFLOW = -8
 LAYOUT_NN, LAYOUT_NT, LAYOUT_TN = 0, 1, 2
 TILE_AUTO = -1
 TILES = {"auto": -1, "256x128": 0, "128x128": 1, "128x64": 2, "64x64": 3, "32x32": 4, "128x128k32": 5, "64x64k16": 6,
-         "256x256": 7, "256x256s": 8, "256x128s": 9, "128x128s": 10, "128x64s": 11, "conv128x128s": 12, "conv64x128s": 13}
+         "256x256": 7, "256x256s": 8, "256x128s": 9, "128x128s": 10, "128x64s": 11, "128x128sc": 12,
+         "conv128x128s": 13, "conv64x128s": 14}
 ACT_LINEAR, ACT_RELU, ACT_SIGMOID, ACT_TANH = 0, 1, 2, 3
 
 

@@ -216,8 +216,8 @@ class Context:
 
     def set_gemm_tile(self, tile="auto") -> None:
         """Force one macro tile ("256x128", "128x128", "128x64", "64x64", "32x32", "128x128k32", "64x64k16",
-        "256x256"; split operands on the bf16 matrix cores: "256x256s", "256x128s", "128x128s", "128x64s" and, for
-        convolutions, "conv128x128s", "conv64x128s") or "auto"."""
+        "256x256"; split operands on the bf16 matrix cores: "256x256s", "256x128s", "128x128s", "128x64s", "128x128sc" and,
+        for convolutions, "conv128x128s", "conv64x128s") or "auto"."""
         check(_lib.load().zn_hip_set_gemm_tile(self.handle, _lib.TILES[tile] if isinstance(tile, str) else tile),
               "zn_hip_set_gemm_tile")
 

@@ -68,7 +68,8 @@ ZN_GEMM_R_UNALIGNED(nn, true, false)
 ZN_GEMM_R_UNALIGNED(nt, true, true)
 ZN_GEMM_R_UNALIGNED(tn, false, false)
 // zn_sgemm_<layout>_s<tile>: operands split into bf16 parts (gemm_split.h),
-// any alignment.  sw: no flushed partial sums, whose registers would spill.
+// any alignment.  sw: no flushed partial sums, whose registers would spill;
+// sc: the same sums on 128x128 tiles.
 // sr: two workgroups to a CU (4096 x 2048 x 1024 NN 95.8 -> 88.4 us, NT 92.4
 // -> 88.8; one round of tiles the same).
 #define ZN_GEMM_SPLIT(NAME, NW, FM, BN, AK, BKC, FLUSH, GC, AB, NV, MINB)                        \
@@ -85,6 +86,7 @@ ZN_GEMM_SPLIT_TILE(sw, 8, 2, 256, false, 1, 1, 5, 2)
 ZN_GEMM_SPLIT_TILE(sx, 8, 2, 128, true, 1, 2, 3, 2)
 ZN_GEMM_SPLIT_TILE(sr, 8, 1, 128, true, 1, 2, 3, 4)
 ZN_GEMM_SPLIT_TILE(sn, 4, 2, 64, true, 2, 2, 3, 2)
+ZN_GEMM_SPLIT_TILE(sc, 8, 1, 128, false, 1, 2, 3, 4)
 
 ZN_GEMM_TILE(h, gemm_tile_pinned, 64, 64, 16, 2, 2, 2)
 

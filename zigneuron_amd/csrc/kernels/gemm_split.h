@@ -31,7 +31,9 @@ namespace {
 //    to the tile's sums, one rounding of the long sum per 32 of K instead of
 //    six (K 512: 1.2e-7 against 3.4e-7).  The 256x256 tile has no registers
 //    for it (it spills 240 of them) and keeps one chain, itself a little
-//    closer to 64 bits than the fp32 kernels.
+//    closer to 64 bits than the fp32 kernels.  Tiles of one kind give a value
+//    the same bits, so the 128x128 one has a chain form too (sc), for a part
+//    of a product whose whole runs on 256x256.
 //  * What bounds it: issue.  A 16x16x32 product takes 18 clocks of its SIMD,
 //    but four vector instructions beside it make that 29 (measured, two waves
 //    a SIMD), and each value costs 6.5 of them to split.  Larger tiles split
@@ -40,7 +42,9 @@ namespace {
 //    slices ahead, XCD-blocked tile orders and four columns at a time changed
 //    nothing.
 //  * Sums that are not finite: the wave does its tile again on the fp32
-//    matrix cores (plain), about five times slower.
+//    matrix cores (plain), about five times slower.  Its finite values then
+//    have that arithmetic's bits; taking only the others from there changes
+//    how the main loop is scheduled (NN and NT on 128x128 2 to 3% slower).
 template <int NW, int FM, int BN, bool AK, bool BKC, bool FLUSH, int GC, int AB, int NV, int G = kGNone, bool GU = false>
 struct SplitTile {
     static constexpr int NT = NW * kWave;

@@ -47,9 +47,9 @@ static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
 namespace {
 
 // Macro tiles of the GEMM code object (kernels/gemm_f32.hip).
-// The last six run on the bf16 matrix cores (three-way split operands,
+// The last seven run on the bf16 matrix cores (three-way split operands,
 // kernels/gemm_split.h); cr and ch are the convolutions'.
-enum Tile { kTileX = 0, kTileL, kTileN, kTileM, kTileS, kTileR, kTileH, kTileW, kTileSW, kTileSX, kTileSR, kTileSN, kTileCR, kTileCH, kNumTiles };
+enum Tile { kTileX = 0, kTileL, kTileN, kTileM, kTileS, kTileR, kTileH, kTileW, kTileSW, kTileSX, kTileSR, kTileSN, kTileSC, kTileCR, kTileCH, kNumTiles };
 struct TileShape {
     int bm, bn, bk, threads;
     const char *suffix;
@@ -69,6 +69,7 @@ constexpr TileShape kTiles[kNumTiles] = {{256, 128, 16, 512, "x", true, true, tr
                                          {256, 128, 32, 512, "sx", false, false, true},
                                          {128, 128, 32, 512, "sr", false, false, true},
                                          {128, 64, 32, 256, "sn", false, false, true},
+                                         {128, 128, 32, 512, "sc", false, false, true},
                                          {128, 128, 32, 512, "cr", false, false, false},
                                          {64, 128, 32, 256, "ch", false, false, false}};
 constexpr const char *kLayoutName[3] = {"nn", "nt", "tn"};
@@ -633,12 +634,19 @@ int choose_splits(const zn_ctx *ctx, Tile tile, int64_t m, int64_t n, int64_t k,
     return splits < 2 ? 1 : (int)splits;
 }
 
-// The split kernels (kernels/gemm_split.h, tiles sw, sx, sr and sn): each
+// The split kernels (kernels/gemm_split.h, tiles sw, sx, sr, sn and sc): each
 // operand value as three bf16 numbers, six bf16 products per fp32 product.
+// Unsplit in K, the tiles of one kind of sum give a value the same bits.
 struct SplitChoice {
-    Tile tile = kTileSR;
+    Tile tile = kTileSR;  // kNumTiles: the fp32 kernels
     int splits = 1;       // K slices
     double us = 0.0;      // estimated time
+};
+constexpr SplitChoice kF32Kernels = {kNumTiles, 1, 0.0};
+enum Sums {
+    kSumsAny,    // whichever tile is the fastest: sw, sx, sr or sn
+    kSumsFlush,  // six products at a time, then added to the sum: sx, sr, sn
+    kSumsChain,  // one chain: sw, and sc for parts of a product whose whole runs on sw
 };
 
 // Estimated time of a problem on one split tile: its workgroups on the
@@ -646,17 +654,21 @@ struct SplitChoice {
 // slice, both as measured on MI355X (us a slice: sw 4.1, sx 2.4, sr 1.5, sn
 // 1.05 alone and 1.6 two at a time), plus a round's start and stores and,
 // for K in slices, the reduce launch.
-SplitChoice estimate_split(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch, int64_t max_ws) {
+SplitChoice estimate_split(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch, int64_t max_ws,
+                           Sums sums = kSumsAny) {
     struct Cost {
         Tile tile;
         double one, two;
         bool pairs;
     };
-    static const Cost kCosts[] = {{kTileSW, 4.1, 0, false}, {kTileSX, 2.4, 0, false}, {kTileSR, 1.5, 0, false}, {kTileSN, 1.05, 1.6, true}};
+    static const Cost kCosts[] = {{kTileSW, 4.1, 0, false}, {kTileSX, 2.4, 0, false}, {kTileSR, 1.5, 0, false},
+                                  {kTileSN, 1.05, 1.6, true}, {kTileSC, 1.5, 0, false}};
     const int64_t cus = cus_now(ctx);
     SplitChoice best;
     best.us = 1e30;
     for (const Cost &c : kCosts) {
+        const bool chain = c.tile == kTileSW || c.tile == kTileSC;
+        if (sums == kSumsAny ? c.tile == kTileSC : (sums == kSumsChain) != chain) continue;
         const int64_t tiles = cdiv(m, kTiles[c.tile].bm) * cdiv(n, kTiles[c.tile].bn) * batch;
         for (int64_t s = 1; s <= 16 && (s == 1 || (k / s >= 512 && 4.0 * s * batch * m * n <= (double)max_ws)); ++s) {
             const double slices = (double)cdiv(cdiv(k, 32), s);
@@ -769,12 +781,13 @@ struct RowTail {
 
 // split_rows: the launch may cut itself into two launches (a row tail; the
 // last problems of a batch), whose calls pass false.
-// arith: 0 the fp32 kernels, 1 the split kernels, -1 whichever pays.
+// given: the split tile and K slices of a part of a larger problem, or
+// kF32Kernels; null leaves them to the policy.
 int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, const float *a, int64_t lda,
                    int64_t stride_a, const float *b, int64_t ldb, int64_t stride_b, float *c, int64_t ldc,
                    int64_t stride_c, int64_t batch, int accumulate, const float *bias, int act, int bias_rows,
                    const ZnConvGeom *conv = nullptr, GatherMode mode = kGatherIm2col, bool split_rows = true,
-                   int padded = 0, RowTail *row_tail = nullptr, int arith = -1) {
+                   int padded = 0, RowTail *row_tail = nullptr, const SplitChoice *given = nullptr) {
     if (!ctx) return ZN_ERR_INVALID_ARG;
     if (layout < ZN_LAYOUT_NN || layout > ZN_LAYOUT_TN) return ZN_ERR_INVALID_ARG;
     if (act < ZN_ACT_LINEAR || act > ZN_ACT_TANH) return ZN_ERR_INVALID_ARG;
@@ -842,7 +855,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // The split kernels: a forced tile, or by size (forced wave splits and persistent kernels are fp32 forms)
     const bool by_size = !forced && k > 0 && ctx->forced_wave_split <= 0 && ctx->forced_persistent < 0;
     const bool bf16x3 = !conv && (forced ? tile >= kTileSW
-                                         : by_size && (arith == 1 || (arith < 0 && split_pays(ctx, m, n, k, batch))));
+                                         : by_size && (given ? given->tile != kNumTiles : split_pays(ctx, m, n, k, batch)));
     int policy_splits = 1;
     const bool conv_policy = conv && !forced && ctx->forced_splits == 0 && ctx->forced_persistent < 0 && k > 0;
     bool conv_split = conv && forced && tile >= kTileCR;
@@ -863,17 +876,16 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
         }
     }
     if (bf16x3 && !forced) {
-        // part of a larger problem: the sums of the whole, which K slices would change
-        SplitChoice ch = estimate_split(ctx, m, n, k, batch, arith == 1 ? 0 : (int64_t)kScratchBytes);
-        const int64_t m_main = split_main_rows(ctx, m, n, k, batch, ch);
+        SplitChoice ch = given ? *given : estimate_split(ctx, m, n, k, batch, (int64_t)kScratchBytes);
+        const int64_t m_main = given ? m : split_main_rows(ctx, m, n, k, batch, ch);
         if (split_rows && m_main < m && ctx->forced_splits == 0) {
             const float *a_tail = layout == ZN_LAYOUT_TN ? a + m_main : a + m_main * lda;
             const int rc = gemm_launch_ex(ctx, layout, m_main, n, k, a, lda, 0, b, ldb, 0, c, ldc, 0, 1, accumulate, bias, act,
-                                          bias_rows, nullptr, mode, false, padded, nullptr, 1);
+                                          bias_rows, nullptr, mode, false, padded, nullptr, &ch);
             if (rc) return rc;
             return gemm_launch_ex(ctx, layout, m - m_main, n, k, a_tail, lda, 0, b, ldb, 0, c + m_main * ldc, ldc, 0, 1, accumulate,
                                   bias && bias_rows ? bias + m_main : bias, act, bias_rows, nullptr, mode, false, padded,
-                                  nullptr, 0);
+                                  nullptr, &kF32Kernels);
         }
         tile = ch.tile;
         policy_splits = ch.splits;
@@ -899,11 +911,11 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
             // the first part may compute the tail rows too (below); if not, they are a second launch
             RowTail tail = {a_tail, c + m_main * ldc, m - m_main, false};
             int rc = gemm_launch_ex(ctx, layout, m_main, n, k, a, lda, 0, b, ldb, 0, c, ldc, 0, 1, accumulate, bias,
-                                    act, bias_rows, nullptr, mode, false, padded, &tail, 0);
+                                    act, bias_rows, nullptr, mode, false, padded, &tail, &kF32Kernels);
             if (rc || tail.folded) return rc;
             return gemm_launch_ex(ctx, layout, m - m_main, n, k, a_tail, lda, 0, b, ldb, 0, c + m_main * ldc, ldc, 0, 1,
                                   accumulate, bias && bias_rows ? bias + m_main : bias, act, bias_rows, nullptr, mode,
-                                  false, padded, nullptr, 0);
+                                  false, padded, nullptr, &kF32Kernels);
         }
     }
     // The 128x128 register-staged tile loads rows that are not whole float4s
@@ -1214,7 +1226,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
         if (splits > 1 && nb == 1) part.xcd_remap = 2;  // the tiles of one K slice share an XCD's L2
         // split 128-row tiles: each XCD a contiguous run of them, which share
         // A panels (4096 x 1024 x 1024 NN 50.1 -> 48.9 us, NT 48.2 -> 46.9)
-        else if (bf16x3 && splits == 1 && nb == 1 && (tile == kTileSR || tile == kTileSN) && ntiles % 8 == 0)
+        else if (bf16x3 && splits == 1 && nb == 1 && (tile == kTileSR || tile == kTileSN || tile == kTileSC) && ntiles % 8 == 0)
             part.xcd_remap = 1;
         part.a = a ? a + b0 * stride_a : nullptr;
         part.b = b ? b + b0 * stride_b : nullptr;
@@ -1533,9 +1545,12 @@ int transfer_step(zn_ctx *ctx, const std::vector<Span> &ups, const std::vector<S
 // i + 1 when accumulating) goes up while the context stream multiplies
 // chunk i and C chunk i - 1 comes down on the download stream (PCIe is full
 // duplex; transfer_step interleaves the two directions).  Each chunk is an
-// ordinary GEMM of `rows` rows on the device buffers, so the row results are
-// those of the unchunked call whenever both run unsplit (split-K changes only
-// the order of K partial sums).
+// ordinary GEMM of `rows` rows on the device buffers, on the kernels that the
+// unchunked call takes for those rows (fp32 ones or split operands, and there
+// the same kind of sum), so the row results are those of the unchunked call
+// whenever both run unsplit (split-K changes only the order of K partial sums)
+// and every sum is finite (a wave of the split kernels that holds one that is
+// not repeats its own 16 or 32 rows on the fp32 matrix cores).
 int host_gemm_chunked(zn_ctx *ctx, int layout, const float *a, const float *b, const float *bias, float *c, size_t m,
                       size_t n, size_t k, int accumulate, int act, float *da, float *db, float *dc, float *dbias,
                       size_t rows) {
@@ -1562,15 +1577,26 @@ int host_gemm_chunked(zn_ctx *ctx, int layout, const float *a, const float *b, c
             {(char *)(c + first(i) * n), (const char *)(dc + first(i) * n), count(i) * n * sizeof(float)}};
     };
     const int64_t ldb = layout == ZN_LAYOUT_NT ? (int64_t)k : (int64_t)n;
-    const int arith = split_pays(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1) ? 1 : 0;  // the whole call's, for every chunk
+    // the unchunked call's kernels: split operands for the first m_main rows (none: 0), the fp32 ones for the others
+    int64_t m_main = 0;
+    Sums sums = kSumsAny;
+    if (split_pays(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1)) {
+        SplitChoice whole = estimate_split(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1, (int64_t)kScratchBytes);
+        m_main = ctx->forced_splits == 0 ? split_main_rows(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1, whole) : (int64_t)m;
+        sums = whole.tile == kTileSW ? kSumsChain : kSumsFlush;
+    }
+    auto multiply = [&](int64_t r0, int64_t rows_, const SplitChoice &with, bool split_rows) {
+        return gemm_launch_ex(ctx, layout, rows_, (int64_t)n, (int64_t)k, da + r0 * (int64_t)k, (int64_t)k, 0, db, ldb, 0,
+                              dc + r0 * (int64_t)n, (int64_t)n, 0, 1, accumulate, bias ? dbias : nullptr, act, 0, nullptr,
+                              kGatherIm2col, split_rows, 0, nullptr, &with);
+    };
     if ((rc = transfer_step(ctx, ups(0), {}))) return rc;
     ZN_HIP_TRY(ctx, hipEventRecord(ctx->chunk_in[0], ctx->up));
     for (size_t i = 0; i < chunks; ++i) {
         ZN_HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, ctx->chunk_in[i & 1], 0));
-        rc = gemm_launch_ex(ctx, layout, (int64_t)count(i), (int64_t)n, (int64_t)k, da + first(i) * k, (int64_t)k, 0, db,
-                            ldb, 0, dc + first(i) * n, (int64_t)n, 0, 1, accumulate, bias ? dbias : nullptr, act, 0,
-                            nullptr, kGatherIm2col, true, 0, nullptr, arith);
-        if (rc) return rc;
+        const int64_t r0 = (int64_t)first(i), main = std::min<int64_t>(std::max<int64_t>(m_main - r0, 0), (int64_t)count(i));
+        if (main > 0 && (rc = multiply(r0, main, estimate_split(ctx, main, (int64_t)n, (int64_t)k, 1, 0, sums), false))) return rc;
+        if (main < (int64_t)count(i) && (rc = multiply(r0 + main, (int64_t)count(i) - main, kF32Kernels, m_main == 0))) return rc;
         ZN_HIP_TRY(ctx, hipEventRecord(ctx->chunk_out[i & 1], ctx->stream));
         if (i >= 1) ZN_HIP_TRY(ctx, hipStreamWaitEvent(ctx->down, ctx->chunk_out[(i - 1) & 1], 0));
         if ((rc = transfer_step(ctx, i + 1 < chunks ? ups(i + 1) : std::vector<Span>{},
