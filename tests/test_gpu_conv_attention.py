@@ -561,10 +561,12 @@ def test_col2im_both_kernels(ctx, channels):
 
 
 @pytest.mark.parametrize("batch,seq,d", [(1, 1000, 80), (1, 2048, 64), (2, 321, 128), (1, 63, 33), (3, 257, 96),
-                                         (1, 255, 1), (70, 130, 64), (1, 4097, 32)])
+                                         (1, 255, 1), (70, 130, 64), (1, 4097, 32), (28, 384, 64), (28, 385, 64),
+                                         (24, 300, 48), (40, 300, 64), (40, 300, 63), (64, 513, 64), (86, 513, 64)])
 def test_attention_key_ranges(ctx, batch, seq, d):
-    """Few problems: the keys go to ranges of their own and zn_attention_combine merges them (and the shapes on either
-    side of that rule); within the bound of the fused walk."""
+    """Few problems: the keys go to ranges of their own and zn_attention_combine merges them; and the shapes on either
+    side of the rules for that and for the fp32 kernels (up to 256 positions of up to 64 dims; 33 to 64 dims that give the
+    split form's larger workgroups no fewer rounds of the CUs); within the bound of the fused walk."""
     rng = np.random.default_rng(seq + d)
     q, k, v = (uniform(rng, (batch, seq, d)) for _ in range(3))
     scale = 1.0 / np.sqrt(d)

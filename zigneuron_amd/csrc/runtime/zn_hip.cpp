@@ -3168,13 +3168,10 @@ int zn_hip_attention_forward(zn_ctx *ctx, const float *q, const float *k, const 
     int rc = select_device(ctx);
     if (rc) return rc;
     const int64_t sd = seq_len * d_k, ss = seq_len * seq_len;
-    // Short sequences of narrow heads stay on the fp32 kernels, whose smaller
-    // workgroups start sooner (MI355X: 128 x 128 x 64 13.6 us, split 17.0; 32
-    // x 192 x 64 17.3 and 22.7; 64 x 256 x 32 13.0 and 13.4; from 512 on the
-    // split form is 1.5 times as fast, and above 64 head dims always faster).
-    if (d_k <= kAttnDims[1] && seq_len <= 256) {
-        const int dim = d_k <= kAttnDims[0] ? 0 : 1;
-        const int vec = d_k % 4 == 0 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out);
+    if (d_k <= kAttnSplitDims[3] && sd <= (int64_t)INT_MAX / 4 && cdiv(seq_len, kAttnQueries) <= 65535) {
+        const int dim = (int)(d_k - 1) / 32;
+        const bool vec = d_k % 4 == 0 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out);
+        const int64_t cus = cus_now(ctx);
         ZnAttnArgs a;
         std::memset(&a, 0, sizeof(a));
         a.stride = sd;
@@ -3182,33 +3179,43 @@ int zn_hip_attention_forward(zn_ctx *ctx, const float *q, const float *k, const 
         a.d_k = (int32_t)d_k;
         a.scale_log2 = scale * 1.44269504088896340736f;
         constexpr int64_t kMaxGridX = (int64_t)1 << 30;
-        for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridX) {
-            const int64_t nb = batch - b0 < kMaxGridX ? batch - b0 : kMaxGridX;
-            ZnAttnArgs c = a;
-            c.q = q + b0 * sd;
-            c.k = k + b0 * sd;
-            c.v = v + b0 * sd;
-            c.out = out + b0 * sd;
-            if ((rc = launch(ctx, ctx->attn[dim][vec], (unsigned)nb, (unsigned)cdiv(seq_len, kAttnQueries), 256, &c))) return rc;
-        }
-        return ZN_OK;
-    }
-    if (d_k <= kAttnSplitDims[3] && sd <= (int64_t)INT_MAX / 4 && cdiv(seq_len, kAttnQueries) <= 65535) {
-        const int dim = (int)(d_k - 1) / 32;
-        ZnAttnArgs a;
-        std::memset(&a, 0, sizeof(a));
-        a.stride = sd;
-        a.seq_len = (int32_t)seq_len;
-        a.d_k = (int32_t)d_k;
-        a.scale_log2 = scale * 1.44269504088896340736f;
         // grid.x = problem (so one problem's query blocks share an XCD), grid.y = query block
-        const int64_t gy = cdiv(seq_len, kAttnSplitQueries[dim]);
+        const int64_t gy32 = cdiv(seq_len, kAttnQueries), gy = cdiv(seq_len, kAttnSplitQueries[dim]);
         // Query blocks for at most a quarter of the CUs: ranges of keys (of at
         // least 64) for the idle ones, merged by a second launch (MI355X, one
         // head of 1000 x 80: 159 us in 8 workgroups of the fp32 kernel, 19.6
         // us in 8 x 16 here; 64 x 256 x 32, two ranges: 15.2 -> 22.8 us).
-        int64_t splits = std::min<int64_t>({32, cdiv(seq_len, 64), cus_now(ctx) / (batch * gy)});
+        int64_t splits = std::min<int64_t>({32, cdiv(seq_len, 64), cus / (batch * gy)});
         if (splits < 4) splits = 1;
+        // Short sequences of narrow heads stay on the fp32 kernels, whose
+        // smaller workgroups start sooner (MI355X: 128 x 128 x 64 13.6 us,
+        // split 17.0; 32 x 192 x 64 17.3 and 22.7; 64 x 256 x 32 13.0 and
+        // 13.4).  So do heads of 33 to 64 dims (16-byte I/O) whose 128-query
+        // fp32 workgroups take hardly more rounds of the CUs than the split
+        // form's 256-query ones: half of those queries are then empty or half
+        // of the CUs idle, and a round of 300 positions takes 33 us split, 26
+        // us fp32 (40 x 300 x 64: 32.8 and 26.2 us; 32 x 768 x 64: 65.2 and
+        // 58.0; 86 x 640 x 64, two rounds of either: 105 and 90.5; three
+        // rounds for two: 180 x 300 x 64 62.2 and 71.5; two for one: 64 x 600
+        // x 64 55.9 and 88.8), up to 2047 positions (16 x 2048 x 64 148 and
+        // 147; 8 x 4096 x 64 283 and 290).  Four key ranges pay from 385 positions on (28
+        // x 300 x 64 30.5 and 26.1 us, 32 x 385 x 64 34.8 and 35.4), five or
+        // more always (24 x 300 x 64 26.0 and 26.1).
+        const int64_t rounds32 = cdiv(batch * gy32, cus), rounds = cdiv(batch * gy, cus);
+        const bool f32 = (dim <= 1 && seq_len <= 256) ||
+                         (dim == 1 && vec && (splits > 1 ? splits < 5 && seq_len <= 384 : seq_len < 2048 && 4 * rounds32 <= 5 * rounds));
+        if (f32) {
+            for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridX) {
+                const int64_t nb = batch - b0 < kMaxGridX ? batch - b0 : kMaxGridX;
+                ZnAttnArgs c = a;
+                c.q = q + b0 * sd;
+                c.k = k + b0 * sd;
+                c.v = v + b0 * sd;
+                c.out = out + b0 * sd;
+                if ((rc = launch(ctx, ctx->attn[dim][vec], (unsigned)nb, (unsigned)gy32, 256, &c))) return rc;
+            }
+            return ZN_OK;
+        }
         const int64_t keys = cdiv(cdiv(seq_len, splits), 32) * 32;
         splits = cdiv(seq_len, keys);
         if (splits > 1 && ensure_workspace(ctx, (size_t)(batch * seq_len * splits * (((d_k + 3) & ~3) + 4)) * sizeof(float)) != ZN_OK)
@@ -3216,7 +3223,6 @@ int zn_hip_attention_forward(zn_ctx *ctx, const float *q, const float *k, const 
         a.splits = (int32_t)splits;
         a.keys_per_split = splits > 1 ? (int32_t)keys : (int32_t)seq_len;
         a.part = ctx->ws;
-        constexpr int64_t kMaxGridX = (int64_t)1 << 30;
         for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridX) {
             const int64_t nb = batch - b0 < kMaxGridX ? batch - b0 : kMaxGridX;
             ZnAttnArgs c = a;
