@@ -543,12 +543,19 @@ def test_c5_conv_backward_properties(ctx):
         assert np.all(np.abs(gi[b] - ref) <= tol(9 * OC) * den * 1.01 + 1e-6), f"image {b}"
 
 
-@pytest.mark.parametrize("channels", [47, 48, 49])
-def test_col2im_both_kernels(ctx, channels):
-    """Around the channel count where zn_col2im (lanes along channels) takes over from zn_col2im_px (lanes along
+@pytest.mark.parametrize("B,H,W,ker,stride,channels",
+                         [(2, 9, 67, 3, (2, 1), 47), (2, 9, 67, 3, (2, 1), 48),  # fewer than 8 blocks of 256 pixels
+                          (1, 3, 5, 3, (1, 1), 7),
+                          (2, 37, 67, 3, (1, 1), 47),                            # few rows of 64 pixels for the chip
+                          (9, 53, 17, 3, (1, 1), 20), (9, 53, 17, 3, (1, 1), 21),
+                          (9, 53, 17, 3, (2, 2), 36), (9, 53, 17, 3, (2, 2), 37),
+                          (9, 53, 17, 5, (2, 2), 26), (9, 53, 17, 5, (2, 2), 27),
+                          (9, 53, 18, 5, (2, 2), 25)])                           # two groups of blocks, the last not full
+def test_col2im_both_kernels(ctx, B, H, W, ker, stride, channels):
+    """Around the channel counts where zn_col2im (lanes along channels) takes over from zn_col2im_px (lanes along
     pixels): both bit-identical to the reference's order."""
-    B, H, W, KH, KW, st, pd = 2, 9, 67, 3, 3, (2, 1), (1, 1)
-    OH, OW = (H + 2 - KH) // 2 + 1, (W + 2 - KW) // 1 + 1
+    KH, KW, st, pd = ker, ker, stride, (ker // 2, ker // 2)
+    OH, OW = (H + 2 * pd[0] - KH) // st[0] + 1, (W + 2 * pd[1] - KW) // st[1] + 1
     rng = np.random.default_rng(channels)
     col = uniform(rng, (B * OH * OW, KH * KW * channels))
     dcol, dout = ctx.to_device(col), ctx.alloc(B * channels * H * W).fill(np.nan)

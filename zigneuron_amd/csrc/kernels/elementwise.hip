@@ -269,18 +269,30 @@ extern "C" __global__ __launch_bounds__(256) void zn_col2im(ZnIm2colArgs p) {
 
 // The same sums, one thread per input element with lanes along the pixels of
 // a row: for few channels, where zn_col2im's channel lanes would idle
-// (MI355X, 16 x 3 x 64 x 64 under 5x5 stride 2: 43.1 us there).
+// (MI355X, 16 x 3 x 64 x 64 under 5x5 stride 2: 43.1 us there).  A workgroup
+// takes 256 pixels of one channel.  Neighbouring channels share their lines of
+// col, so a group of blocks goes through its channels one after the other, and
+// each block stays on the XCD (workgroups go round the 8 of them) whose L2
+// holds its lines: px_group is a multiple of 8 with up to 2 MiB of col for
+// each XCD (29 x 20 x 40 x 40 under 5x5: 199 us in the order of the images, 82
+// so; 32 x 12 x 61 x 61 321 and 111).
 extern "C" __global__ __launch_bounds__(256) void zn_col2im_px(ZnIm2colArgs p) {
     const int kc = p.k_h * p.k_w * p.channels;
     const int64_t hw = (int64_t)p.out_h * p.out_w;
-    const int64_t total = (int64_t)p.batch * p.channels * p.in_h * p.in_w;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int64_t bch = i / p.in_w;
-        const int iw = (int)(i - bch * p.in_w);
-        const int64_t bc = bch / p.in_h;
-        const int ih = (int)(bch - bc * p.in_h);
-        const int64_t b = bc / p.channels;
-        const int ic = (int)(bc - b * p.channels);
+    const int64_t pixels = (int64_t)p.batch * p.in_h * p.in_w;
+    const uint32_t plane = (uint32_t)p.in_h * (uint32_t)p.in_w, channels = (uint32_t)p.channels;
+    // the images have at most 2^36 elements in memory, so the workgroups fit 32 bits
+    const uint32_t blocks = (uint32_t)((pixels + 255) / 256), group = (uint32_t)p.px_group;
+    const uint32_t units = (blocks + group - 1) / group * group * channels;
+    for (uint32_t u = blockIdx.x; u < units; u += gridDim.x) {
+        const uint32_t r = u / group, q = r / channels;
+        const int ic = (int)(r - q * channels);
+        const int64_t first = (int64_t)(q * group + (u - r * group)) * 256;  // the workgroup's first pixel
+        if (first + threadIdx.x >= pixels) continue;
+        const int64_t image = first >> 32 ? first / plane : (uint32_t)first / plane;
+        const uint32_t at = (uint32_t)(first - image * plane) + threadIdx.x, next = at / plane, row = (at - next * plane) / (uint32_t)p.in_w;
+        const int64_t b = image + next;
+        const int ih = (int)row, iw = (int)(at - next * plane - row * (uint32_t)p.in_w);
         const int hh = ih + p.pad_h, ww = iw + p.pad_w;
         const int oh_lo = hh >= p.k_h ? (hh - p.k_h) / p.stride_h + 1 : 0;
         const int oh_hi = min(hh / p.stride_h, p.out_h - 1);
@@ -297,7 +309,7 @@ extern "C" __global__ __launch_bounds__(256) void zn_col2im_px(ZnIm2colArgs p) {
                 sum = sum + cb[((int64_t)oh * p.out_w + ow) * kc + tap];
             }
         }
-        p.image[i] = sum;
+        p.image[((b * p.channels + ic) * p.in_h + ih) * p.in_w + iw] = sum;
     }
 }
 

@@ -2394,13 +2394,47 @@ static ZnIm2colArgs col_args(float *image, float *col, int64_t batch, int64_t c,
     a.pad_h = (int32_t)ph;
     a.pad_w = (int32_t)pw;
     a.k_order = k_order;
+    a.px_group = 0;
     return a;
 }
 
 // zn_im2col: one workgroup per tile of 64 col rows x 64 taps; zn_col2im: one
-// per 64 pixels of an input row (grid-stride loops cover the rest), or below
-// kCol2imChannels channels one thread per input element (zn_col2im_px).
-constexpr int kCol2imChannels = 48;
+// per 64 pixels of an input row (grid-stride loops cover the rest), or for few
+// channels one thread per input element (zn_col2im_px).  The first takes about
+// the same time up to 64 channels, the second grows with them.  Where they
+// meet (MI355X, us of zn_col2im and zn_col2im_px, batches of 4 to 32 images of
+// 25 to 128 pixels a side):
+//  * first kernel's workgroups for less than 1.75 a CU: px up to 47 channels
+//    (8 x 40 x 40 under 3x3 with 47 channels 29/27, 2 x 112 x 112 under 5x5
+//    with 40 channels 119/106), and above
+//  * col in im2col order: 8 or more taps to a pixel up to 20 channels (28 x 44
+//    x 44 under 3x3 with 16, 20, 24 channels 39/33, 39/41, 40/49; under 5x5
+//    92/73, 92/95, 93/116); 1.5 to 4 up to 36 (3x3 stride 2 with 32, 40
+//    channels: 32 x 61 x 61 41/38, 42/48); else up to 26 (5x5 stride 2 with 24,
+//    28 channels 35/32, 36/39); up to 2 workgroups a CU 12 more, but for 8 to
+//    16 taps (16 x 32 x 32 under 5x5 with 32, 40 channels 64/53, 64/69, under
+//    3x3 with 24, 32 channels 16/16, 17/21); 1x1 up to 26, or 40 below 3.5
+//    workgroups a CU (28 x 44 x 44 with 24, 32 channels 13/12, 13/15; 28 x 29 x
+//    29 with 40, 47 channels 10/9, 10/10);
+//  * in OIHW order the first kernel's channel lanes lie a filter apart
+//    themselves (the whole backward with 17 outputs): 8 to 16 taps to a pixel
+//    up to 28 channels (3x3 with 28, 32, 40 channels, 16 x 64 x 64: 191/190,
+//    216/220, 233/254), 1x1 as above, else up to 47 (5x5 with 47: 1092/774).
+static bool col2im_by_pixels(const zn_ctx *ctx, const ZnIm2colArgs &a) {
+    const int64_t taps = (int64_t)a.k_h * a.k_w, step = (int64_t)a.stride_h * a.stride_w;  // taps / step of them to a pixel
+    const int64_t units = a.batch * (int64_t)a.in_h * cdiv(a.in_w, 64), cus = cus_now(ctx);
+    const bool middle = taps >= 8 * step && taps < 16 * step;
+    int most = 47;
+    if (4 * units > 7 * cus) {
+        if (2 * taps < 3 * step)
+            most = 2 * units <= 7 * cus ? 40 : 26;
+        else if (a.k_order == 0)
+            most = (taps >= 8 * step ? 20 : taps < 4 * step ? 36 : 26) + (units <= 2 * cus && !middle ? 12 : 0);
+        else if (middle)
+            most = 28;
+    }
+    return a.channels <= std::min(most, 47);
+}
 static int im2col_launch(zn_ctx *ctx, const ZnIm2colArgs &a) {
     const int rc = select_device(ctx);
     if (rc) return rc;
@@ -2415,8 +2449,14 @@ static int col2im_launch(zn_ctx *ctx, const ZnIm2colArgs &a) {
     if (rc) return rc;
     const int64_t cap = cus_now(ctx) * 32;
     ZnIm2colArgs c = a;
-    if (a.channels < kCol2imChannels) {
-        const int64_t blocks = std::min<int64_t>(cdiv((int64_t)a.batch * a.channels * a.in_h * a.in_w, 256), cap);
+    if (col2im_by_pixels(ctx, a)) {
+        // equal groups, of a multiple of 8 blocks with at most 2 MiB of col for each XCD; fewer than 8 blocks are one group
+        const int64_t px_blocks = cdiv((int64_t)a.batch * a.in_h * a.in_w, 256);
+        const int64_t most = 8 * std::max<int64_t>(1, 2048 / ((int64_t)a.k_h * a.k_w * a.channels));
+        const int64_t even = cdiv(px_blocks, cdiv(px_blocks, most));
+        const int64_t group = px_blocks < 8 ? px_blocks : cdiv(even, 8) * 8;
+        c.px_group = (int32_t)group;
+        const int64_t blocks = std::min<int64_t>(cdiv(px_blocks, group) * group * a.channels, cap);
         return launch(ctx, ctx->elt[kCol2imPx], (unsigned)blocks, 1, 256, &c);
     }
     const int64_t units = (int64_t)a.batch * a.in_h * cdiv(a.in_w, 64);

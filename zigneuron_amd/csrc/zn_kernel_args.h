@@ -212,6 +212,7 @@ struct ZnIm2colArgs {
     float *col;    // written by im2col, read by col2im
     int32_t batch, channels, in_h, in_w, k_h, k_w, out_h, out_w, stride_h, stride_w, pad_h, pad_w;
     int32_t k_order;
+    int32_t px_group;  // zn_col2im_px: blocks of 256 pixels that take each channel in turn
 };
 
 // Row packing: dst[r][c] = c < cols ? src[r * ld_src + c] : 0 for
