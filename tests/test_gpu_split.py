@@ -229,6 +229,20 @@ def test_chunked_host_call_has_the_bits_of_the_device_call(ctx, m, n, k):
     backend.deinit()
 
 
+def test_chunked_host_call_of_few_rows_and_long_k(ctx):
+    """1024 x 1000 x 8195 in chunks of 256 rows, whose few tiles split K: K slices of whole 32s, the last one with a tail."""
+    from zigneuron_amd import Backend
+    m, n, k = 1024, 1000, 8195
+    rng = np.random.default_rng(23)
+    a, b = uniform(rng, (m, k)), uniform(rng, (k, n))
+    announce(f"chunked host call {m}x{n}x{k}")
+    backend = Backend.init(0)
+    host = np.empty((m, n), np.float32)
+    backend.matMul(a, b, host, m, n, k)
+    backend.deinit()
+    check_rows(host, "nn", a, b, k, np.r_[0:m:61, m - 1], "chunked")
+
+
 CONVS = [(4, 64, 56, 56, 128, 3, 1, 1),   # channels a multiple of 32: one tap per K slice
          (16, 36, 33, 35, 100, 3, 1, 1),  # taps change inside a slice; rows of 35 pixels
          (16, 32, 61, 59, 48, 5, 2, 2),   # stride 2, 64-row tiles
