@@ -545,7 +545,6 @@ struct AttnSplit {
 
 ZN_ATTN_DIM(32, 64)
 ZN_ATTN_DIM(64, 64)
-ZN_ATTN_DIM(128, 32)
 
 // zn_attention_s<DP>: the split form, head dims up to DP, any alignment;
 // NW waves of FQ x 16 queries.

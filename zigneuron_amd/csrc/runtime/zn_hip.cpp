@@ -88,7 +88,7 @@ constexpr const char *kEltObject = "zn_elementwise_gfx950.hsaco";
 constexpr const char *kMlpObject = "zn_mlp_gfx950.hsaco";
 constexpr const char *kAttnObject = "zn_attention_gfx950.hsaco";
 // Fused attention kernels by padded head dim (zn_attention_d<dim>[_v]).
-constexpr int kAttnDims[3] = {32, 64, 128};
+constexpr int kAttnDims[2] = {32, 64};
 constexpr int kAttnQueries = 128;  // queries per workgroup (4 waves x 32)
 // The split form (zn_attention_s<dim>): padded head dims, threads and queries of a workgroup.
 constexpr int kAttnSplitDims[4] = {32, 64, 96, 128};
@@ -173,7 +173,7 @@ struct zn_ctx {
     hipFunction_t pair_fwd[2] = {};            // fused two-layer Dense forward [16-byte staging]
     int pair_fwd_threads[2] = {};              // its workgroup size (the kernel's launch bounds)
     hipFunction_t pair_bwd[4][2][2] = {};      // fused two-layer Dense backward [lower act][non-linear head][16-byte]
-    hipFunction_t attn[3][2] = {};             // fused attention [head dim 32/64/128][16-byte I/O]
+    hipFunction_t attn[2][2] = {};             // fused attention [head dim 32/64][16-byte I/O]
     hipFunction_t attn_split[4] = {};          // the split form [head dim 32/64/96/128]
     hipFunction_t attn_combine = nullptr;      // merges its key ranges
     hipFunction_t gemm[3][kNumTiles][3] = {};  // [layout][tile][staging: 4-byte, 16-byte, 16-byte unaligned (r only)]
@@ -532,7 +532,8 @@ int launch_reduce(zn_ctx *ctx, ZnReduceArgs &r) {
 // workgroups; below that, 64x64 tiles (4 waves) are the fastest down to the
 // smallest problems and for N <= 64 (C5 P.V: 169 us against 184 us for
 // 128x64), except for exactly one round of 128x128 tiles (below); 32x32 and
-// 128x64 tiles never beat them and are left to explicit selection.  A tile
+// 128x64 tiles never beat them, and problems large enough for 256x256 run on
+// split operands: these are left to explicit selection.  A tile
 // whose padding wastes more than a quarter of its MFMA work (for example
 // 256-row tiles over M = 128) is skipped for the next smaller one.
 // A gathered (implicit convolution) operand costs more per staged element, so
@@ -543,13 +544,6 @@ Tile choose_tile(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t bat
     const int64_t cus = cus_now(ctx);
     auto tiles = [&](Tile t) { return cdiv(m, kTiles[t].bm) * cdiv(n, kTiles[t].bn) * batch; };
     auto useful = [&](Tile t) { return 4 * m * n * batch >= 3 * tiles(t) * kTiles[t].bm * kTiles[t].bn; };
-    // 256x256 (16-byte staging only, one workgroup per CU): long K and whole
-    // rounds of tiles, the last at least 80% full (8192^3 NN 141.7 -> 145.4
-    // TFLOP/s, 4096^3 125.5 -> 133.7 against 256x128; a ragged last round
-    // would leave CUs idle for a whole 256x256 tile)
-    if (wide_ok && k >= 512 && tiles(kTileW) >= cus && useful(kTileW) &&
-        5 * tiles(kTileW) >= 4 * cdiv(tiles(kTileW), cus) * cus)
-        return kTileW;
     // short K: a tile's epilogue outweighs its K walk, and the smaller l tile
     // overlaps them better (C5 QK^T, K = 64: l 242 us, x 252 us, round-robin
     // A/B); up to K = 128 its persistent kernels take the problem
@@ -1967,7 +1961,7 @@ int zn_hip_create(int device, const char *code_object_dir, zn_ctx **out) {
                 if (hipModuleGetFunction(&ctx->pair_bwd[a1][a2][v], ctx->mlp_module, name) != hipSuccess)
                     return bail(ZN_ERR_SYMBOL);
             }
-    for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < 2; ++d)
         for (int v = 0; v < 2; ++v) {
             char name[64];
             std::snprintf(name, sizeof(name), "zn_attention_d%d%s", kAttnDims[d], v ? "_v" : "");
