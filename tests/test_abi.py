@@ -92,11 +92,21 @@ def test_code_objects_hold_every_kernel():
         assert k.encode() in gemm
     for k in ("zn_fill_f32", "zn_copy_f32", "zn_add_bias", "zn_activation_forward", "zn_activation_backward",
               "zn_accumulate_bias", "zn_im2col", "zn_softmax_rows", "zn_col2im", "zn_row_sum", "zn_dense_grad_prologue",
-              "zn_hold_stream"):
+              "zn_hold_stream", "zn_col2im_px", "zn_reduce_slices"):
         assert k.encode() in elt
-    for d in (32, 64, 128):
+    for d in (32, 64):
         for v in ("", "_v"):
             assert f"zn_attention_d{d}{v}".encode() in attn
+    # split operands on the bf16 matrix cores
+    for lay in ("nn", "nt", "tn"):
+        for t in ("sw", "sx", "sr", "sn", "sc"):
+            assert f"zn_sgemm_{lay}_{t}\0".encode() in gemm
+    for fam in ("zn_convfs_nt", "zn_convts_nt", "zn_convwns_tn"):
+        for t in ("cr", "ch"):
+            for u in ("", "_u"):
+                assert f"{fam}_{t}{u}\0".encode() in conv
+    for k in ("s32", "s64", "s96", "s128", "combine"):
+        assert f"zn_attention_{k}\0".encode() in attn
     for k in ("zn_dense_pair_fwd", "zn_dense_pair_fwd_v"):
         assert k.encode() in mlp
     for a1 in range(4):
