@@ -379,11 +379,13 @@ def test_graph_replay_of_mlp_step_matches_eager(ctx, pair):
         b.close()
 
 
-def test_graph_replay_of_large_tiles_matches_eager(ctx):
+@pytest.mark.parametrize("tiles", [("256x256", "128x128k32", "128x128k32"), ("auto", "auto", "auto")], ids=["fp32", "policy"])
+def test_graph_replay_of_large_tiles_matches_eager(ctx, tiles):
     """The register-staged tiles under graph capture: a 256x256-tile GEMM
     (4096 x 4096 x 512), whole rounds of 128x128 tiles (4096 x 2048 x 256)
     and one round of 128x128 tiles in 4 K slices with the split-K reduce
-    (C3's 1024 x 1024 x 4096 TN), captured once and replayed three times
+    (C3's 1024 x 1024 x 4096 TN), and what the policy takes for them (split
+    operands; the last in K slices), captured once and replayed three times
     with outputs poisoned and unrelated eager GEMMs in between: every replay
     reproduces the eager results bit for bit."""
     rng = np.random.default_rng(17)
@@ -395,10 +397,12 @@ def test_graph_replay_of_large_tiles_matches_eager(ctx):
         bufs.append((lay, m, n, k, a, b, ctx.alloc(m * n), m if lay == "tn" else k))
 
     def run():
-        for lay, m, n, k, a, b, c, lda in bufs:
+        for (lay, m, n, k, a, b, c, lda), tile in zip(bufs, tiles):
+            ctx.set_gemm_tile(tile)
             ctx.sgemm(lay, m, n, k, a, lda, b, n, c, n)
+        ctx.set_gemm_tile("auto")
 
-    announce("graph replay of large tiles")
+    announce(f"graph replay of large tiles {tiles[0]}")
     run()
     ctx.sync()
     eager = [c.download() for *_, c, _ in bufs]

@@ -588,10 +588,12 @@ def test_attention_key_ranges(ctx, batch, seq, d):
         b.close()
 
 
-@pytest.mark.parametrize("batch,seq,d", [(1, 700, 64), (40, 200, 64), (1, 300, 100)])
+@pytest.mark.parametrize("batch,seq,d", [(1, 700, 64), (40, 200, 64), (1, 300, 100), (40, 200, 100), (40, 75, 128),
+                                         (40, 300, 32), (64, 600, 64), (5, 700, 64)])
 def test_attention_non_finite_and_huge(ctx, batch, seq, d):
     """Scores of -inf (a key whose product with every query is -inf gets weight 0), a NaN key, and values of 1e30 (whose
-    scaled parts overflow): what fp32 arithmetic gives, on the queries they reach and on the others."""
+    scaled parts overflow): what fp32 arithmetic gives, on the queries they reach and on the others.  All but 40 x 200 x 64
+    run on split operands, with one range of keys (from 40 heads on) or several, on each of the four kernels."""
     rng = np.random.default_rng(seq)
     q, k, v = (np.abs(uniform(rng, (batch, seq, d))) + np.float32(0.1) for _ in range(3))
     k[0, 5] = -np.inf            # weight 0 for every query

@@ -1,11 +1,13 @@
 """GPU checks of the GEMMs on the bf16 matrix cores (zn_sgemm_<layout>_s*,
-operands split into three bf16 parts): problems of 2^30 multiply-adds and
-more with K of 256 or more, Backend.matMul and its transposes
-(src/backend.zig:169-325).
+operands split into three bf16 parts) and of the convolutions on them:
+Backend.matMul and its transposes (src/backend.zig:169-325).  The policy takes
+them for part of the problems of 2^30 multiply-adds and more with K of 256 or
+more; the tests name each tile (zn_hip_set_gemm_tile), at small extents, and
+take the policy's choice at large ones.
 
-- sampled rows of every layout against fp64 within 2e-7 * sqrt(K) of the
-  componentwise bound (five times tighter than the fp32 kernels' bar), at
-  extents one below and above the tiles' and at K tails of 1 to 31;
+- every layout against fp64 within 2e-7 * sqrt(K) of the componentwise bound
+  (a fiftieth of the fp32 kernels' bar), at extents one below and above the
+  tiles' and at K tails of 1 to 31;
 - values near the ends of the fp32 range, where unscaled parts would be
   subnormal, keep that bound;
 - Inf, NaN and sums beyond 2^80 give what fp32 arithmetic gives;
@@ -13,6 +15,8 @@ more with K of 256 or more, Backend.matMul and its transposes
   bases and strided batches.
 """
 from __future__ import annotations
+
+import contextlib
 
 import numpy as np
 import pytest
@@ -29,6 +33,20 @@ def ctx():
     c = Context(0)
     yield c
     c.close()
+
+
+TILES = ["256x256s", "256x128s", "128x128s", "128x64s", "128x128sc"]
+
+
+@contextlib.contextmanager
+def forced(ctx, tile, splits=0):
+    ctx.set_gemm_tile(tile)
+    ctx.set_gemm_splits(splits)
+    try:
+        yield
+    finally:
+        ctx.set_gemm_tile("auto")
+        ctx.set_gemm_splits(0)
 
 
 def as_mk(a, layout):
@@ -49,24 +67,40 @@ def check_rows(out, layout, a, b, k, rows, what):
     assert np.isfinite(out).all() and err.max() <= 2e-7 * np.sqrt(k), f"{what}: {err.max():.3g}"
 
 
-SHAPES = [(4097, 1023, 777),    # 128x128 rows and a one-row tail
-          (4096, 1025, 257),    # one column past the tiles, K tail of 1
-          (2049, 2047, 287),    # K tail of 31
-          (4100, 4097, 288),    # a column past 32 tiles, whole K slices
-          (1025, 1023, 1027),   # 128x64 tiles
-          (300, 260, 16389),    # K in slices with the reduce
-          (8192, 131, 1030)]
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k,splits", [(257, 129, 33, 0),    # one row and column past the tiles; K tails of 1 ...
+                                          (255, 191, 287, 0),   # ... and 31
+                                          (128, 256, 64, 0),    # whole tiles and K slices
+                                          (3, 5, 31, 0),        # less than a slice
+                                          (300, 260, 1029, 3)])  # K split in three with the reduce
+def test_split_tile_against_fp64(ctx, layout, tile, m, n, k, splits):
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a_shape, b_shape = stored_shapes(layout, m, n, k)
+    a, b = uniform(rng, a_shape), uniform(rng, b_shape)
+    announce(f"split {tile} {layout} {m}x{n}x{k} splits {splits}")
+    with forced(ctx, tile, splits):
+        out = run_gemm(ctx, layout, a, b, m, n, k)
+    check_rows(out, layout, a, b, k, np.arange(m), f"{tile} {layout} {m}x{n}x{k}")
+
+
+SHAPES = [(4097, 1023, 777),    # split 128x128 tiles, and one row on the fp32 kernels
+          (4096, 1025, 257),    # fp32: one column past the tiles
+          (4100, 4097, 288),    # split 256x128 tiles
+          (300, 260, 16389),    # fp32 in K slices
+          (1024, 1000, 8195)]   # split 256x128 tiles in K slices
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("m,n,k", SHAPES)
-def test_split_against_fp64(ctx, layout, m, n, k):
+def test_policy_against_fp64(ctx, layout, m, n, k):
+    """Problems around the line between the split and the fp32 kernels, which stay within the same bound here."""
     rng = np.random.default_rng(m + 3 * n + 7 * k)
     a_shape, b_shape = stored_shapes(layout, m, n, k)
     a, b = uniform(rng, a_shape), uniform(rng, b_shape)
     announce(f"split {layout} {m}x{n}x{k}")
     rows = np.unique(np.r_[0, 1, m // 2, np.arange(max(0, m - 130), m, 7), m - 1])
-    check_rows(run_gemm(ctx, layout, a, b, m, n, k), layout, a, b, k, rows, f"split {layout} {m}x{n}x{k}")
+    check_rows(run_gemm(ctx, layout, a, b, m, n, k), layout, a, b, k, rows, f"policy {layout} {m}x{n}x{k}")
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
@@ -81,15 +115,17 @@ def test_split_largest_tile(ctx, layout):
 
 
 @pytest.mark.parametrize("scale_a,scale_b", [(2e-38, 1.0), (1.0, 2e-38), (1e-30, 1e30), (1e28, 1e-20)])
-def test_split_keeps_small_values(ctx, scale_a, scale_b):
+@pytest.mark.parametrize("tile", TILES)
+def test_split_keeps_small_values(ctx, tile, scale_a, scale_b):
     """Elements at the lower end of the fp32 range (their third parts would be subnormal bf16 numbers unscaled)."""
-    m, n, k = 2049, 2047, 287
+    m, n, k = 391, 277, 287
     rng = np.random.default_rng(9)
     a = (uniform(rng, (m, k)) * np.float32(scale_a)).astype(np.float32)
     b = (uniform(rng, (k, n)) * np.float32(scale_b)).astype(np.float32)
-    announce(f"split range {scale_a} {scale_b}")
-    out = run_gemm(ctx, "nn", a, b, m, n, k)
-    rows = np.arange(0, m, 97)
+    announce(f"split range {tile} {scale_a} {scale_b}")
+    with forced(ctx, tile):
+        out = run_gemm(ctx, "nn", a, b, m, n, k)
+    rows = np.arange(m)
     a64, b64 = a[rows].astype(np.float64), b.astype(np.float64)
     err = np.abs(out[rows] - a64 @ b64)
     # results below 2^-126 round to multiples of 2^-149
@@ -97,19 +133,21 @@ def test_split_keeps_small_values(ctx, scale_a, scale_b):
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
-def test_split_non_finite_and_huge(ctx, layout):
+@pytest.mark.parametrize("tile,splits", [(t, 0) for t in TILES] + [("256x256s", 3), ("128x128s", 3)])
+def test_split_non_finite_and_huge(ctx, layout, tile, splits):
     """Inf, NaN and sums past 2^80 (where the scaled split overflows): the same values as fp32 arithmetic, and the rows
     and columns they do not touch stay within the bound."""
-    m, n, k = 2049, 2047, 287
+    m, n, k = 1001, 1030, 287
     rng = np.random.default_rng(10)
     a, b = np.abs(uniform(rng, (m, k))) + np.float32(0.1), np.abs(uniform(rng, (k, n))) + np.float32(0.1)
-    a[5, 7], a[130, k - 1], a[700, 0], a[2048, 3] = np.inf, np.nan, -np.inf, np.float32(3e38)
+    a[5, 7], a[130, k - 1], a[700, 0], a[m - 1, 3] = np.inf, np.nan, -np.inf, np.float32(3e38)
     a[900] *= np.float32(1e30)  # finite in fp32: 1e30 * 300
     b[11, 40], b[2, 1000] = np.inf, np.nan
     ast = np.ascontiguousarray(a.T) if layout == "tn" else a
     bst = np.ascontiguousarray(b.T) if layout == "nt" else b
-    announce(f"split non-finite {layout}")
-    out = run_gemm(ctx, layout, ast, bst, m, n, k)
+    announce(f"split non-finite {tile} {layout} splits {splits}")
+    with forced(ctx, tile, splits):
+        out = run_gemm(ctx, layout, ast, bst, m, n, k)
     with np.errstate(all="ignore"):
         ref = a.astype(np.float64) @ b.astype(np.float64)
         ref32 = np.where(np.abs(ref) > np.finfo(np.float32).max, np.sign(ref) * np.inf, ref)
@@ -121,22 +159,25 @@ def test_split_non_finite_and_huge(ctx, layout):
 
 
 @pytest.mark.parametrize("act", ["linear", "relu", "sigmoid", "tanh"])
-def test_split_epilogues(ctx, act):
-    m, n, k = 2049, 2047, 260
+@pytest.mark.parametrize("tile,splits", [(t, 0) for t in TILES] + [("128x128s", 2)])
+def test_split_epilogues(ctx, act, tile, splits):
+    m, n, k = 391, 277, 260
     rng = np.random.default_rng(12)
     a, b, bias = uniform(rng, (m, k)), uniform(rng, (k, n)), uniform(rng, (n,))
-    announce(f"split epilogue {act}")
-    out = run_gemm(ctx, "nn", a, b, m, n, k, bias=bias, act=act)
-    rows = np.r_[0:2049:113, 2048]
+    announce(f"split epilogue {tile} {act} splits {splits}")
+    with forced(ctx, tile, splits):
+        out = run_gemm(ctx, "nn", a, b, m, n, k, bias=bias, act=act)
+    rows = np.r_[0:m:13, m - 1]
     assert_close(out[rows], ref_gemm("nn", np.ascontiguousarray(a[rows]), b, len(rows), n, k, bias=bias, act=act), "nn",
                  np.ascontiguousarray(a[rows]), b, len(rows), n, k, bias=bias, act=act, what=f"split {act}")
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
-def test_split_padded_rows_accumulate_batches(ctx, layout):
+@pytest.mark.parametrize("tile", TILES)
+def test_split_padded_rows_accumulate_batches(ctx, layout, tile):
     """Leading dimensions and bases off 16 bytes, accumulation, NaN in the row padding (never read as a value), and a
     strided batch with a shared B."""
-    m, n, k, batch = 1025, 515, 273, 8
+    m, n, k, batch = 259, 131, 73, 5
     rng = np.random.default_rng(13)
     a_shape, b_shape = stored_shapes(layout, m, n, k)
     lda, ldb, ldc = a_shape[1] + 3, b_shape[1] + 1, n + 5
@@ -151,13 +192,14 @@ def test_split_padded_rows_accumulate_batches(ctx, layout):
     da = ctx.to_device(np.concatenate([[0.0], a.ravel()]).astype(np.float32))
     db = ctx.to_device(b)
     dc = ctx.to_device(np.concatenate([[0.0], c0.ravel()]).astype(np.float32))
-    announce(f"split padded batch {layout}")
-    ctx.sgemm_strided_batched(layout, m, n, k, da.offset(1), lda, sa, db, ldb, 0, dc.offset(1), ldc, sc, batch, True)
+    announce(f"split padded batch {tile} {layout}")
+    with forced(ctx, tile):
+        ctx.sgemm_strided_batched(layout, m, n, k, da.offset(1), lda, sa, db, ldb, 0, dc.offset(1), ldc, sc, batch, True)
     out = dc.download()[1:].reshape(batch, sc)
     for i in range(batch):
         view, old = (x[i, :m * ldc].reshape(m, ldc) for x in (out, c0))
         np.testing.assert_array_equal(view[:, n:], old[:, n:])
-        rows = np.r_[0:m:101, m - 1]
+        rows = np.arange(m)
         a64, b64 = as_mk(av[i], layout)[rows].astype(np.float64), as_kn(bv, layout).astype(np.float64)
         ref = old[rows, :n] + a64 @ b64
         den = np.abs(old[rows, :n]) + np.abs(a64) @ np.abs(b64)
@@ -243,20 +285,20 @@ def test_chunked_host_call_of_few_rows_and_long_k(ctx):
     check_rows(host, "nn", a, b, k, np.r_[0:m:61, m - 1], "chunked")
 
 
-CONVS = [(4, 64, 56, 56, 128, 3, 1, 1),   # channels a multiple of 32: one tap per K slice
-         (16, 36, 33, 35, 100, 3, 1, 1),  # taps change inside a slice; rows of 35 pixels
-         (16, 32, 61, 59, 48, 5, 2, 2),   # stride 2, 64-row tiles
-         (2, 128, 40, 40, 200, 3, 1, 0),  # no padding, 38 pixels a row
-         (33, 64, 28, 28, 64, 3, 1, 1),
-         (16, 32, 63, 63, 128, 3, 2, 1)]  # stride 2 with whole fours of pixels a row
+CONVS = [(3, 64, 20, 28, 96, 3, 1, 1),   # channels of 32: one tap per K slice; rows of whole fours of pixels (the _u kernels)
+         (3, 36, 21, 19, 100, 3, 1, 1),  # taps change inside a slice; rows of 19 pixels
+         (5, 32, 31, 29, 48, 5, 2, 2),   # stride 2
+         (2, 64, 22, 22, 40, 3, 1, 0),   # no padding
+         (2, 4, 17, 16, 4, 3, 1, 1)]     # fewer channels than a tile's rows, K of little more than a slice
+TILED = [(c, t) for c in CONVS for t in ("conv128x128s", "conv64x128s")]
 
 
-@pytest.mark.parametrize("case", CONVS)
+@pytest.mark.parametrize("case,tile", TILED + [((16, 32, 63, 63, 128, 3, 2, 1), "auto")])
 @pytest.mark.parametrize("poison", [False, True])
-def test_split_convolutions(ctx, case, poison):
-    """The convolution forward and backward (im2col branch, src/backend.zig:3881-4065) of 2^29 multiply-adds and more
-    against fp64 on the reference's im2col; poison: an Inf in the input and a NaN in grad_output reach exactly the
-    results they reach in fp64."""
+def test_split_convolutions(ctx, case, tile, poison):
+    """The convolution forward and backward (im2col branch, src/backend.zig:3881-4065) on each tile of the split kernels,
+    against fp64 on the reference's im2col; poison: an Inf in the input and a NaN in grad_output reach exactly the results
+    they reach in fp64.  The kernels taken: test_forced_convolution_tiles."""
     from oracle import oracle
     B, C, H, W, OC, ker, st, pd = case
     OH, OW = (H + 2 * pd - ker) // st + 1, (W + 2 * pd - ker) // st + 1
@@ -269,9 +311,10 @@ def test_split_convolutions(ctx, case, poison):
     dx, dw, db, dg = (ctx.to_device(a) for a in (x, w, bias, g))
     y, gx, gw, gb = (ctx.alloc(n).fill(0.5) for n in (B * OC * OH * OW, x.size, w.size, OC))
     geom = (B, C, OC, ker, ker, H, W, OH, OW, st, st, pd, pd)
-    announce(f"split convolution {case} poison {poison}")
-    ctx.conv2d_forward_im2col(dx, dw, db, y, *geom)
-    ctx.conv2d_backward_im2col(dx, dw, dg, gx, gw, gb, *geom)
+    announce(f"split convolution {case} {tile} poison {poison}")
+    with forced(ctx, tile):
+        ctx.conv2d_forward_im2col(dx, dw, db, y, *geom)
+        ctx.conv2d_backward_im2col(dx, dw, dg, gx, gw, gb, *geom)
     col = oracle.im2col(x, B, C, H, W, ker, ker, stride=(st, st), pad=(pd, pd)).reshape(B * OH * OW, -1).astype(np.float64)
     w64, g64 = w.astype(np.float64), g.astype(np.float64)
 
@@ -299,6 +342,31 @@ def test_split_convolutions(ctx, case, poison):
                 den[at] += dcol[sl].reshape(B, OH, OW, C)
         inner = np.s_[:, pd:pd + H, pd:pd + W]
         check(gx.download().reshape(B, C, H, W).transpose(0, 2, 3, 1), ref[inner], den[inner], taps // C * OC, "input gradient")
+    for b in (dx, dw, db, dg, y, gx, gw, gb):
+        b.close()
+
+
+@pytest.mark.parametrize("case", [CONVS[0], CONVS[1]])
+def test_forced_convolution_tiles(ctx, case):
+    """Forward, input and weight gradient take the forced kernels: unsplit in K, both split tiles give the same bits and
+    the fp32 64x64 tile others."""
+    B, C, H, W, OC, ker, st, pd = case
+    OH, OW = (H + 2 * pd - ker) // st + 1, (W + 2 * pd - ker) // st + 1
+    rng = np.random.default_rng(31)
+    x, w, bias, g = (uniform(rng, n) for n in ((B, C, H, W), (OC, ker * ker * C), (OC,), (B * OH * OW, OC)))
+    dx, dw, db, dg = (ctx.to_device(v) for v in (x, w, bias, g))
+    y, gx, gw, gb = (ctx.alloc(n) for n in (B * OC * OH * OW, x.size, w.size, OC))
+    geom = (B, C, OC, ker, ker, H, W, OH, OW, st, st, pd, pd)
+    out = {}
+    for tile in ("conv128x128s", "conv64x128s", "64x64"):
+        announce(f"forced convolution {case} {tile}")
+        with forced(ctx, tile, 1):
+            ctx.conv2d_forward_im2col(dx, dw, db, y, *geom)
+            ctx.conv2d_backward_im2col(dx, dw, dg, gx, gw, gb, *geom)
+        out[tile] = [v.download().view(np.uint32) for v in (y, gx, gw)]
+    for i, what in enumerate(("forward", "input gradient", "weight gradient")):
+        np.testing.assert_array_equal(out["conv128x128s"][i], out["conv64x128s"][i], err_msg=what)
+        assert not np.array_equal(out["conv128x128s"][i], out["64x64"][i]), what
     for b in (dx, dw, db, dg, y, gx, gw, gb):
         b.close()
 
