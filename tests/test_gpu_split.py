@@ -234,6 +234,19 @@ def test_forced_tile_takes_the_named_kernel(ctx, layout):
     assert not np.array_equal(out["128x128"], out["auto"])
 
 
+@pytest.mark.parametrize("m,n,k,split", [(1792, 1536, 1024, False), (3200, 768, 1024, False), (2176, 1408, 832, False), (3520, 896, 1280, True)])
+def test_transposed_product_below_a_round_of_split_tiles(ctx, m, n, k, split):
+    """Whole float4s, TN, 128x128 tiles for 59 to 77% of the CUs: on the fp32 kernels where their 64x64 tiles fill a round,
+    by the bits."""
+    rng = np.random.default_rng(24)
+    a, b = uniform(rng, (k, m)), uniform(rng, (k, n))
+    announce(f"tn policy {m}x{n}x{k}")
+    auto = run_gemm(ctx, "tn", a, b, m, n, k)
+    with forced(ctx, "128x128s" if split else "64x64", 1):
+        np.testing.assert_array_equal(auto.view(np.uint32), run_gemm(ctx, "tn", a, b, m, n, k).view(np.uint32))
+    check_rows(auto, "tn", a, b, k, np.r_[0:m:97, m - 1], "tn policy")
+
+
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("tiles", [("256x256s", "128x128sc"), ("256x128s", "128x128s", "128x64s")], ids=["chain", "flush"])
 def test_split_tiles_agree_bit_for_bit(ctx, layout, tiles):

@@ -698,14 +698,24 @@ int64_t split_main_rows(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int6
 // mostly stores), and so is less than 2^30 multiply-adds, where one round of
 // 64x64 fp32 tiles is as fast (MI355X, 1000^3: 24.1 us split, 24.3 us fp32).
 // Above, the estimate is set against what the fp32 kernels reach: about 125
-// TFLOP/s with 128x128 tiles for most of the CUs, 95 below.
-bool split_pays(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch) {
+// TFLOP/s with 128x128 tiles for most of the CUs, 95 below.  There the TN
+// product of whole float4s is nearer to both: its operands take 16-byte loads
+// on the fp32 kernels and dwords here (1.1 of the estimate), and 64x64 tiles
+// that fill most of a round of three a CU reach 110 (1792 x 1536 x 1024 fp32
+// 53.5 us, split 56.7; 2176 x 1408 x 832 45.3 and 48.0; 3200 x 768 x 1024 53.3
+// and 56.4; in 2.1 rounds of them 3520 x 896 x 1280 74.8 and 69.9).
+bool split_pays(const zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, int64_t batch) {
     const double macs = (double)m * n * k * batch;
     if (k < 256 || macs < 1073741824.0) return false;
-    const double f32_us = 2e-6 * macs / (20 * cdiv(m, 128) * cdiv(n, 128) * batch >= 17 * cus_now(ctx) ? 125.0 : 95.0);
+    const int64_t cus = cus_now(ctx);
     SplitChoice c = estimate_split(ctx, m, n, k, batch, (int64_t)kScratchBytes);
     (void)split_main_rows(ctx, m, n, k, batch, c);
-    return c.us < f32_us;
+    if (20 * cdiv(m, 128) * cdiv(n, 128) * batch >= 17 * cus) return c.us < 2e-6 * macs / 125.0;
+    if (layout == ZN_LAYOUT_TN && m % 4 == 0 && n % 4 == 0 && c.tile == kTileSR && c.splits == 1) {
+        const int64_t tiles64 = cdiv(m, 64) * cdiv(n, 64) * batch;
+        return 1.1 * c.us < 2e-6 * macs / (5 * tiles64 >= 12 * cus && tiles64 <= 3 * cus ? 110.0 : 98.0);
+    }
+    return c.us < 2e-6 * macs / 95.0;
 }
 
 // The tile a gathered convolution GEMM (M rows, N columns, `batch` images)
@@ -849,7 +859,7 @@ int gemm_launch_ex(zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, con
     // The split kernels: a forced tile, or by size (forced wave splits and persistent kernels are fp32 forms)
     const bool by_size = !forced && k > 0 && ctx->forced_wave_split <= 0 && ctx->forced_persistent < 0;
     const bool bf16x3 = !conv && (forced ? tile >= kTileSW
-                                         : by_size && (given ? given->tile != kNumTiles : split_pays(ctx, m, n, k, batch)));
+                                         : by_size && (given ? given->tile != kNumTiles : split_pays(ctx, layout, m, n, k, batch)));
     int policy_splits = 1;
     const bool conv_policy = conv && !forced && ctx->forced_splits == 0 && ctx->forced_persistent < 0 && k > 0;
     bool conv_split = conv && forced && tile >= kTileCR;
@@ -1574,7 +1584,7 @@ int host_gemm_chunked(zn_ctx *ctx, int layout, const float *a, const float *b, c
     // the unchunked call's kernels: split operands for the first m_main rows (none: 0), the fp32 ones for the others
     int64_t m_main = 0, max_ws = 0;
     Sums sums = kSumsAny;
-    if (split_pays(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1)) {
+    if (split_pays(ctx, layout, (int64_t)m, (int64_t)n, (int64_t)k, 1)) {
         SplitChoice whole = estimate_split(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1, (int64_t)kScratchBytes);
         m_main = ctx->forced_splits == 0 ? split_main_rows(ctx, (int64_t)m, (int64_t)n, (int64_t)k, 1, whole) : (int64_t)m;
         sums = whole.tile == kTileSW ? kSumsChain : kSumsFlush;
