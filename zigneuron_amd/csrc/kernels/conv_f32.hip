@@ -116,7 +116,8 @@ ZN_CONVWN_TILE(s, gemm_tile_dma, 32, 32, 32, 1, 1, 1)
 // step (C5's weight gradient GEMM 140 -> 128 us: 315 scalar instructions a
 // slice before, 80 now).  cr of the forward and the input gradient: one
 // column block at a time fits 128 registers, two workgroups to a CU (C5's
-// forward GEMM 123 -> 106 us); the weight gradient, one round of workgroups,
+// forward GEMM 123 -> 106 us; without _u 40 bytes spill, three of the values
+// inside the loop); the weight gradient, one round of workgroups,
 // would spill there (217 us), and ch measured the same with either.
 #define ZN_CONV_SPLIT(NAME, NW, AK, BKC, G, GU, GC, MINB)                                        \
     extern "C" __global__ __launch_bounds__(NW * 64, MINB) void NAME(ZnGemmArgs p) {             \

@@ -34,13 +34,17 @@ namespace {
 //    closer to 64 bits than the fp32 kernels.  Tiles of one kind give a value
 //    the same bits, so the 128x128 one has a chain form too (sc), for a part
 //    of a product whose whole runs on 256x256.
-//  * What bounds it: issue.  A 16x16x32 product takes 18 clocks of its SIMD,
-//    but four vector instructions beside it make that 29 (measured, two waves
-//    a SIMD), and each value costs 6.5 of them to split.  Larger tiles split
-//    each value for more products: 256x256 4.2-4.4 ms at 8192^3 (the fp32
-//    tile 7.35), 256x128 4.8, 128x128 5.2, 128x64 6.0.  Loads two and four
-//    slices ahead, XCD-blocked tile orders and four columns at a time changed
-//    nothing.
+//  * What bounds it: the vector instructions beside the products, 6.5 to split
+//    a value and 1.1 a product on 256x256 tiles, 3.1 on 128x128 (a product
+//    alone takes 16 clocks of its matrix core; four vector instructions beside
+//    it made that 29 in a loop of nothing else).  Counters: at 8192^3 the
+//    matrix cores are busy 74% of the time, in one round of 128x128 tiles 35 to
+//    38%.  Larger tiles split each value for more products: 256x256 4.2-4.4 ms
+//    at 8192^3 (the fp32 tile 7.35), 256x128 4.8, 128x128 5.2, 128x64 6.0.
+//    Loads two and four slices ahead, XCD-blocked tile orders and four columns
+//    at a time changed nothing.
+//  * Registers: 256x256 spills 112 bytes around its loop and in the epilogue,
+//    none inside it.
 //  * Sums that are not finite: the wave does its tile again on the fp32
 //    matrix cores (plain), about five times slower.  Its finite values then
 //    have that arithmetic's bits; taking only the others from there changes

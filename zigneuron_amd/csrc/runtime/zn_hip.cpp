@@ -644,10 +644,13 @@ enum Sums {
 };
 
 // Estimated time of a problem on one split tile: its workgroups on the
-// busiest CU (one resident, for sn up to two) times the time of a 32-deep
-// slice, both as measured on MI355X (us a slice: sw 4.1, sx 2.4, sr 1.5, sn
-// 1.05 alone and 1.6 two at a time), plus a round's start and stores and,
-// for K in slices, the reduce launch.
+// busiest CU, one after the other (sn: two at a time), times the time of a
+// 32-deep slice as measured on MI355X (us a slice: sw 4.1, sx 2.4, sr and sc
+// 1.5, sn 1.05 alone and 1.6 two at a time), plus a round's start and stores
+// and, for K in slices, the reduce launch.  Over 58 problems of 2^30 to 2^34.5
+// multiply-adds the estimate is 0.85 to 1.25 of the time: one round of sr 0.85
+// to 1.0 (1.55 us a slice and 5.5), two rounds 1.03 to 1.21 (two of its
+// workgroups share a CU: 1.4 us a slice each), sw 0.88 to 1.25.
 SplitChoice estimate_split(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch, int64_t max_ws,
                            Sums sums = kSumsAny) {
     struct Cost {
@@ -722,7 +725,10 @@ bool split_pays(const zn_ctx *ctx, int layout, int64_t m, int64_t n, int64_t k, 
 // takes on the split kernels, or kNumTiles when the fp32 kernels are kept:
 // less than 2^29 multiply-adds, K below 128, fewer than 33 rows (half the
 // tile padding), or an estimate above the 95 TFLOP/s those reach.  Measured
-// us a slice, one workgroup a CU: cr 1.5, ch 1.0.
+// us a slice, one workgroup a CU: cr 1.5, ch 1.0 (cr of the forward and the
+// input gradient holds two since, which the estimate does not count).  Over 36
+// convolutions of 2^29 to 2^34 multiply-adds no forward or backward is more
+// than 3% slower than with the fp32 kernels alone.
 Tile conv_split_tile(const zn_ctx *ctx, int64_t m, int64_t n, int64_t k, int64_t batch, int64_t splits) {
     const double macs = (double)m * n * k * batch;
     if (k < 128 || m < 33 || macs < 536870912.0) return kNumTiles;
