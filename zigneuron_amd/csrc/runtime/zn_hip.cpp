@@ -2465,7 +2465,8 @@ static int col2im_launch(zn_ctx *ctx, const ZnIm2colArgs &a) {
     if (col2im_by_pixels(ctx, a)) {
         // equal groups, of a multiple of 8 blocks with at most 2 MiB of col for each XCD; fewer than 8 blocks are one group
         const int64_t px_blocks = cdiv((int64_t)a.batch * a.in_h * a.in_w, 256);
-        const int64_t most = 8 * std::max<int64_t>(1, 2048 / ((int64_t)a.k_h * a.k_w * a.channels));
+        const int64_t taps = (int64_t)a.k_h * a.k_w * a.channels, step = (int64_t)a.stride_h * a.stride_w;
+        const int64_t most = 8 * std::max<int64_t>(1, 2048 * step / taps);
         const int64_t even = cdiv(px_blocks, cdiv(px_blocks, most));
         const int64_t group = px_blocks < 8 ? px_blocks : cdiv(even, 8) * 8;
         c.px_group = (int32_t)group;
